@@ -29,12 +29,10 @@
 // kernel adds the splits in order (deterministic) and applies the epilogue.
 #include <math.h>
 
-#include "q4d_device.h"
 #include "q4d_internal.h"
+#include "q4d_mfma_dev.h"
 
 namespace q4d {
-
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
 constexpr int kGemmBN = 128;
 // waves per block for 128- and 64-row tiles
@@ -45,25 +43,6 @@ constexpr int kGemmBK = 64;
 // fastest on the prefill projections (fewer store bank conflicts than 72)
 constexpr int kGemmPad = 16;
 constexpr int kGemmLds = kGemmBK + kGemmPad;
-
-// Dequantise 8 consecutive int4 (one 32-bit word, low nibble first) times `scale` to
-// fp16, in column order: word p of the result holds columns 2p, 2p + 1.
-__device__ __forceinline__ u32x4 dequant8(uint32_t w, h2 scale2) {
-  const h2 bias = make_h2((_Float16)1032.0f, (_Float16)1032.0f);
-  const uint32_t v = w ^ 0x88888888u;
-  const uint32_t lo = v & 0x0F0F0F0Fu;         // nibbles 0, 2, 4, 6 in bytes 0..3
-  const uint32_t hi = (v >> 4) & 0x0F0F0F0Fu;  // nibbles 1, 3, 5, 7
-  u32x4 out;
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    // fp16 pair (nibble 2p, nibble 2p+1): low byte of each half from lo / hi byte p
-    const uint32_t sel = (uint32_t)(p) | (0x0Cu << 8) | ((uint32_t)(4 + p) << 16) | (0x0Cu << 24);
-    const uint32_t pr = __builtin_amdgcn_perm(hi, lo, sel) | 0x64006400u;
-    const h2 q = __builtin_bit_cast(h2, pr) - bias;
-    out[p] = __builtin_bit_cast(uint32_t, q * scale2);
-  }
-  return out;
-}
 
 // Dequantise 32 consecutive int4 (one 16-byte chunk) times `scale` to fp16,
 // in column order.
@@ -789,24 +768,6 @@ constexpr int kSkRows = 16;        // weight rows per block
 constexpr int kSkKW = 128;         // K columns per wave
 constexpr int kSkMaxWaves = 8;     // waves per block at most (K columns per block <= 1024)
 constexpr int kSkRedStride = 68;   // LDS row stride of the partial tiles (floats; conflict-free)
-
-// Word s of lane row group G becomes word G of row group s (lane l % 16 kept).
-// v_permlane32_swap(A, B) returns (A.lo | B.lo, A.hi | B.hi) over lanes 0-31 | 32-63;
-// v_permlane16_swap(A, B) returns (A.r0 | B.r0 | A.r2 | B.r2, A.r1 | B.r1 | A.r3 | B.r3)
-// over the 16-lane rows r0..r3.
-__device__ __forceinline__ void rows_transpose4(uint32_t (&d)[4]) {
-  // the off-diagonal 2 x 2 blocks: rows 0-1 words 2-3 <-> rows 2-3 words 0-1
-  const auto a = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
-  const auto b = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
-  const uint32_t e0 = a[0], e2 = a[1], e1 = b[0], e3 = b[1];
-  // inside each 2 x 2 block: the even rows' odd words <-> the odd rows' even words
-  const auto c = __builtin_amdgcn_permlane16_swap(e0, e1, false, false);
-  const auto f = __builtin_amdgcn_permlane16_swap(e2, e3, false, false);
-  d[0] = c[0];
-  d[1] = c[1];
-  d[2] = f[0];
-  d[3] = f[1];
-}
 
 template <int EP, bool PAIR>
 __global__ __launch_bounds__(kSkMaxWaves * 64) void q4_skinny_kernel(const GemmArgs a) {

@@ -816,6 +816,9 @@ int launch_gemv_xp(const GemvArgs& a, int xm, int xp, int ep, bool pair, hipStre
   if ((a.x_parts || a.x_out) && (ep != EP_ARGMAX || xm != X_RMS || a.cols != 1024 || !a.x_parts)) return Q4D_ERR_SHAPE;
   if ((a.x_parts && !aligned(a.x_parts, 16)) || (a.x_out && !aligned(a.x_out, 16))) return Q4D_ERR_BAD_ADDR;
   if (xm == X_F16 && xp != 1) return Q4D_ERR_DTYPE;
+  // plain linear over several rows: one unpacked weight for 16 of them
+  if (a.batch >= kRowsMin && a.nseg == 1 && !pair && (xm == X_F16 || xm == X_F32) && (ep == EP_F16 || ep == EP_F32))
+    return launch_rows(RowsArgs{a.w[0], a.s[0], a.x, a.y, nullptr, a.batch, a.rows, a.cols}, xm == X_F32, xp, ep, st);
   // unused segments: empty ranges on segment 0's memory, never selected
   GemvArgs b = a;
   if (pair) {
@@ -844,6 +847,13 @@ int launch_gemv_group(int rows, int cols, int batch, const uint8_t* const* w, co
   for (int i = 0; i < count; ++i) {
     if (!w[i] || !s[i] || !x[i] || !y[i]) return Q4D_ERR_NULL;
     if (!aligned(w[i], 16) || !aligned(s[i], 4) || !aligned(x[i], 16)) return Q4D_ERR_BAD_ADDR;
+  }
+  if (batch >= kRowsMin) {  // as q4d_linear: each matrix fills the device by itself
+    for (int i = 0; i < count; ++i) {
+      const int rc = launch_rows(RowsArgs{w[i], s[i], x[i], y[i], nullptr, batch, rows, cols}, xm == X_F32, xp, ep, st);
+      if (rc) return rc;
+    }
+    return Q4D_OK;
   }
   GemvGroupArgs G;
   memset(&G, 0, sizeof(G));

@@ -199,6 +199,24 @@ int launch_gemv(const GemvArgs& a, int xmode, int epmode, bool pair, hipStream_t
 int launch_gemv_group(int rows, int cols, int batch, const uint8_t* const* w, const uint16_t* const* s,
                       const void* const* x, void* const* y, int count, int xm, int xp, int ep, hipStream_t st);
 
+// ---- Q4 linear over several activation rows on MFMA (q4d_rows.hip) -----------
+// y[m] = W x[m] for M rows at the GEMV's precision (xp: 2 = fp32 x as fp16 hi + lo, 1 = one
+// fp16 value); ep EP_F16 / EP_F32, or EP_RESID (fp16 x): y = resid + W x, fp32, resid may
+// alias y.  K % 128 == 0.
+struct RowsArgs {
+  const uint8_t* w;
+  const uint16_t* s;
+  const void* x;       // [M, K] fp32 or fp16
+  void* y;             // [M, N]
+  const float* resid;  // [M, N]
+  int M, N, K;
+};
+int launch_rows(const RowsArgs& a, bool xf32, int xp, int ep, hipStream_t st);
+// Activation rows from which q4d_linear takes this kernel instead of one GEMV per row
+// (3072 x 1024 / 1024 x 3072, fp32: 3 rows 3.7 / 4.5 us as GEMVs; 4 rows 4.0 / 5.0 against
+// 3.2 / 5.1 here, 8 rows 5.8 / 8.0 against 3.2 / 5.1).
+constexpr int kRowsMin = 4;
+
 // ---- other launchers ---------------------------------------------------------
 int launch_rms_norm(const float* x, const float* gamma, float eps, int rows, int dim, void* y,
                     int y_dtype, hipStream_t stream);

@@ -1,0 +1,60 @@
+// Device-side building blocks shared by the Q4 kernels that feed MFMA.
+#pragma once
+
+#include "q4d_device.h"
+
+namespace q4d {
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+
+// 8 consecutive int4 (one 32-bit word, low nibble first) as fp16 integers, in column
+// order: word p of the result holds columns 2p, 2p + 1.  (0x6400 | u) is 1024 + u, so
+// subtracting 1032 gives q = u - 8 exactly.
+__device__ __forceinline__ u32x4 codes8(uint32_t w) {
+  const h2 bias = make_h2((_Float16)1032.0f, (_Float16)1032.0f);
+  const uint32_t v = w ^ 0x88888888u;
+  const uint32_t lo = v & 0x0F0F0F0Fu;         // nibbles 0, 2, 4, 6 in bytes 0..3
+  const uint32_t hi = (v >> 4) & 0x0F0F0F0Fu;  // nibbles 1, 3, 5, 7
+  u32x4 out;
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    // fp16 pair (nibble 2p, nibble 2p+1): low byte of each half from lo / hi byte p
+    const uint32_t sel = (uint32_t)(p) | (0x0Cu << 8) | ((uint32_t)(4 + p) << 16) | (0x0Cu << 24);
+    const uint32_t pr = __builtin_amdgcn_perm(hi, lo, sel) | 0x64006400u;
+    out[p] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, pr) - bias);
+  }
+  return out;
+}
+
+// The same times `scale`: one correctly rounded fp16 multiply per element (the scale code
+// is an exact fp16 below 2048, i.e. scale < 0.125).
+__device__ __forceinline__ u32x4 dequant8(uint32_t w, h2 scale2) {
+  const u32x4 q = codes8(w);
+  u32x4 out;
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const uint32_t qp = q[p];
+    out[p] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, qp) * scale2);
+  }
+  return out;
+}
+
+// Word s of lane row group G becomes word G of row group s (lane l % 16 kept).
+// v_permlane32_swap(A, B) returns (A.lo | B.lo, A.hi | B.hi) over lanes 0-31 | 32-63;
+// v_permlane16_swap(A, B) returns (A.r0 | B.r0 | A.r2 | B.r2, A.r1 | B.r1 | A.r3 | B.r3)
+// over the 16-lane rows r0..r3.
+__device__ __forceinline__ void rows_transpose4(uint32_t (&d)[4]) {
+  // the off-diagonal 2 x 2 blocks: rows 0-1 words 2-3 <-> rows 2-3 words 0-1
+  const auto a = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
+  const uint32_t e0 = a[0], e2 = a[1], e1 = b[0], e3 = b[1];
+  // inside each 2 x 2 block: the even rows' odd words <-> the odd rows' even words
+  const auto c = __builtin_amdgcn_permlane16_swap(e0, e1, false, false);
+  const auto f = __builtin_amdgcn_permlane16_swap(e2, e3, false, false);
+  d[0] = c[0];
+  d[1] = c[1];
+  d[2] = f[0];
+  d[3] = f[1];
+}
+
+}  // namespace q4d

@@ -1,0 +1,249 @@
+// Q4 linear over several activation rows on MFMA, at the GEMV's precision (gfx950).
+//
+//   y[m, n] = sum_g scale[n, g] * sum_{k in group g} q[n, k] x[m, k]      (4 rows and more)
+//
+// The GEMV (q4d_gemv.hip) reads and unpacks every weight again for each activation row: at
+// 211 rows of a 1024 x 3072 matrix its VALU work took 161 us.  Here 16 rows share each
+// unpacked weight.  The arithmetic keeps the GEMV's precision: the int4 codes enter the MFMA
+// as exact fp16 integers, fp32 activations as an fp16 hi + fp16 lo pair (~22 significant
+// bits, two MFMAs; fp16 activations and activation precision 1 take one), products are
+// exact, a 64-column group is summed in fp32 by its own MFMA accumulator and multiplied by
+// its Q2.14 scale in fp32.
+//
+// Work split: a block owns 16 MT activation rows x 16 NT weight rows; its waves split K in
+// units of 128 columns (two scale groups) and their partial tiles are summed through LDS in
+// wave order, so the result is deterministic.  A unit's activations are read as whole
+// 512-byte row pieces, split into hi / lo and laid out for the MFMA in LDS that belongs to
+// the wave alone (no barrier); read straight into the MFMA operand layout, each load
+// instruction would touch 64 separate cache lines.  The codes go to registers: 16 bytes per
+// lane, transposed across the four lane rows as in the skinny GEMM (q4d_gemm.hip).
+//
+// What bounds it: a few rows, the launch and one memory round trip (16 rows of 3072 x 1024
+// fp32: 3.3 us, 9.4 as 16 GEMVs); many, the unpacking and splitting VALU work per MFMA and
+// the activations' re-reads from L2 (211 rows of 1024 x 3072: 9.5 us, was 142; 1024 rows of
+// 3072 x 1024: 34 us, was 466).
+#include "q4d_internal.h"
+#include "q4d_mfma_dev.h"
+
+namespace q4d {
+
+namespace {
+
+constexpr int kRwUnit = 128;           // K columns per wave and step
+constexpr int kRwLd = kRwUnit + 16;    // LDS row stride in fp16: 288 B, conflict-free MFMA operand reads
+constexpr int kRwRed = 17;             // LDS row stride (floats) of the partial tiles
+
+// XF32: fp32 activations (else fp16).  XP: 2 = hi + lo halves, 1 = one fp16 value.  The block's
+// tile is 16 MT activation rows x 16 NT weight rows.  UPW > 0: every wave has UPW units and
+// issues all their loads at entry; 0: any number, the next unit's loads in flight.
+template <bool XF32, int XP, int EP, int MT, int NT, int NW, int UPW>
+__global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
+  static_assert(XF32 || XP == 1, "fp16 activations are one value");
+  constexpr int kX = NW * XP * 16 * MT * kRwLd * 2, kR = NW * MT * NT * 16 * kRwRed * 4;
+  __shared__ __attribute__((aligned(16))) char lds[kX > kR ? kX : kR];
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int nl = lane & 15, G = lane >> 4;
+  const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+  const int nu = a.K / kRwUnit;
+  const int u0 = w * nu / NW, u1 = (w + 1) * nu / NW;
+  _Float16* xs = reinterpret_cast<_Float16*>(lds) + (size_t)w * XP * 16 * MT * kRwLd;
+
+  // rows past the end read the last one; their results are not stored
+  // (32-bit offsets from the block's first rows: one address register per load)
+  const uint8_t* wb = a.w + (size_t)n0 * (a.K / 2);
+  const char* sb = reinterpret_cast<const char*>(a.s) + (size_t)n0 * (a.K / 32);
+  uint32_t wo[NT], so[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const uint32_t n = min(16 * j + nl, a.N - 1 - n0);
+    wo[j] = n * (a.K / 2) + 16 * G;
+    so[j] = n * (a.K / 32);
+  }
+  // activation loads of a unit: XL instructions, each CPR lanes of 16 bytes per row
+  constexpr int XB = XF32 ? 4 : 2, CPR = 8 * XB, RPI = 64 / CPR, XL = 16 * MT / RPI;
+  const int xr = lane / CPR, xc = lane % CPR;
+  const char* xb = static_cast<const char*>(a.x) + (size_t)m0 * a.K * XB;
+  uint32_t xo[XL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) xo[i] = (uint32_t)min(RPI * i + xr, a.M - 1 - m0) * a.K * XB + 16 * xc;
+
+  struct Unit {
+    u32x4 x[XL];
+    u32x4 c[NT];
+    uint32_t s[NT];
+  } U[UPW > 0 ? UPW : 1];
+  auto load = [&](Unit& L, int u) {
+#pragma unroll
+    for (int i = 0; i < XL; ++i) L.x[i] = *reinterpret_cast<const u32x4*>(xb + u * (kRwUnit * XB) + xo[i]);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      L.c[j] = *reinterpret_cast<const u32x4*>(wb + u * (kRwUnit / 2) + wo[j]);
+      L.s[j] = *reinterpret_cast<const uint32_t*>(sb + 4 * u + so[j]);
+    }
+  };
+  f32x4 tot[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) tot[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  auto step = [&](Unit& L, int u) {
+    // activations to LDS: row RPI i + xr, hi at 0, lo 16 MT rows further
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+      _Float16* d = xs + (RPI * i + xr) * kRwLd + xc * (16 / XB);
+      if constexpr (XF32) {
+        uint32_t hw[2], lw[2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const uint32_t b0 = L.x[i][2 * p], b1 = L.x[i][2 * p + 1];
+          const float f0 = __builtin_bit_cast(float, b0), f1 = __builtin_bit_cast(float, b1);
+          const h2 h = make_h2((_Float16)f0, (_Float16)f1);
+          hw[p] = __builtin_bit_cast(uint32_t, h);
+          if constexpr (XP == 2)
+            lw[p] = __builtin_bit_cast(uint32_t, make_h2((_Float16)(f0 - (float)h.x), (_Float16)(f1 - (float)h.y)));
+        }
+        *reinterpret_cast<u32x2*>(d) = u32x2{hw[0], hw[1]};
+        if constexpr (XP == 2) *reinterpret_cast<u32x2*>(d + 16 * MT * kRwLd) = u32x2{lw[0], lw[1]};
+      } else {
+        *reinterpret_cast<u32x4*>(d) = L.x[i];
+      }
+    }
+    uint32_t d4[NT][4], sc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      sc[j] = L.s[j];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d4[j][e] = L.c[j][e];
+    }
+    if (UPW == 0 && u + 1 < u1) load(L, u + 1);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) rows_transpose4(d4[j]);
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      f32x4 p[MT][NT];
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) p[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 2 * g; s < 2 * g + 2; ++s) {
+        h8 xh[MT], xl[MT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          const _Float16* xp = xs + (16 * i + nl) * kRwLd + 32 * s + 8 * G;
+          xh[i] = *reinterpret_cast<const h8*>(xp);
+          if constexpr (XP == 2) xl[i] = *reinterpret_cast<const h8*>(xp + 16 * MT * kRwLd);
+        }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          const h8 q = __builtin_bit_cast(h8, codes8(d4[j][s]));
+#pragma unroll
+          for (int i = 0; i < MT; ++i) {
+            p[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[i], q, p[i][j], 0, 0, 0);
+            if constexpr (XP == 2) p[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[i], q, p[i][j], 0, 0, 0);
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const float f = scale_q2_14(g ? sc[j] >> 16 : sc[j] & 0xFFFFu);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) tot[i][j][r] = fmaf(p[i][j][r], f, tot[i][j][r]);
+      }
+    }
+  };
+  if constexpr (UPW > 0) {
+#pragma unroll
+    for (int d = 0; d < UPW; ++d) load(U[d], u0 + d);
+#pragma unroll
+    for (int d = 0; d < UPW; ++d) step(U[d], u0 + d);
+  } else {
+    if (u0 < u1) load(U[0], u0);
+    for (int u = u0; u < u1; ++u) step(U[0], u);
+  }
+
+  // lane holds activation rows 16 i + 4G + r of weight row 16 j + l % 16
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[(((w * NT + j) * MT + i) * 16 + 4 * G + r) * kRwRed + nl] = tot[i][j][r];
+  __syncthreads();
+  for (int o = t; o < MT * NT * 256; o += NW * 64) {
+    const int c = o % (16 * NT), j = c >> 4, m = o / (16 * NT);
+    if (m0 + m >= a.M || n0 + c >= a.N) continue;
+    float v = red[(j * 16 * MT + m) * kRwRed + (c & 15)];
+#pragma unroll
+    for (int q = 1; q < NW; ++q) v += red[((q * NT + j) * 16 * MT + m) * kRwRed + (c & 15)];
+    const size_t oo = (size_t)(m0 + m) * a.N + n0 + c;
+    if constexpr (EP == EP_F16)
+      static_cast<_Float16*>(a.y)[oo] = (_Float16)v;
+    else if constexpr (EP == EP_RESID)
+      static_cast<float*>(a.y)[oo] = a.resid[oo] + v;
+    else
+      static_cast<float*>(a.y)[oo] = v;
+  }
+}
+
+template <bool XF32, int XP, int EP, int MT, int NT>
+int launch_tile(const RowsArgs& a, hipStream_t st) {
+  const dim3 grid((a.N + 16 * NT - 1) / (16 * NT), (a.M + 16 * MT - 1) / (16 * MT));
+  const auto go = [&](auto kernel, int nw) { hipLaunchKernelGGL(kernel, grid, dim3(64 * nw), 0, st, a); };
+  // Every unit of a wave in flight where K is one of the projections' widths and the
+  // registers hold them (211 x 1024 x 3072, hi + lo: 9.5 us, 11.5 with the next unit only);
+  // K = 3072 on one-tile blocks: 12 waves of two units (4 rows: 5.1 us, 5.5 with 8 of three).
+  constexpr bool kSmall = MT == 1 && NT == 1, kDeep = XP == 1 || MT * NT <= 4;
+  const int nu = a.K / kRwUnit;
+  if (nu == 8)
+    go(rows_kernel<XF32, XP, EP, MT, NT, 8, 1>, 8);
+  else if (nu == 16 && kDeep)
+    go(rows_kernel<XF32, XP, EP, MT, NT, 8, kDeep ? 2 : 0>, 8);
+  else if (nu == 24 && kSmall)
+    go(rows_kernel<XF32, XP, EP, MT, NT, kSmall ? 12 : 8, kSmall ? 2 : 0>, kSmall ? 12 : 8);
+  else if (nu == 24 && kDeep)
+    go(rows_kernel<XF32, XP, EP, MT, NT, 8, kDeep && !kSmall ? 3 : 0>, 8);
+  else
+    go(rows_kernel<XF32, XP, EP, MT, NT, 8, 0>, 8);
+  return check_launch();
+}
+
+template <bool XF32, int XP, int EP>
+int launch_nt(const RowsArgs& a, hipStream_t st) {
+  // The largest tile (each split activation serves NT weight tiles, each unpacked weight MT
+  // row tiles) that still gives most CUs a block: 512 rows of 3072 x 1024, fp16: 24.4 us with
+  // MT = 1, 16.3 with 2; 64 rows of 2048 x 1024: 3.6 us on 256 blocks, 4.8 on 128.
+  const int mt = (a.M + 15) / 16, nt = (a.N + 15) / 16;
+  const auto blocks = [&](int m, int n) { return (long)((mt + m - 1) / m) * ((nt + n - 1) / n); };
+  constexpr long kMinBlocks = 192;
+  if (blocks(2, 4) >= kMinBlocks) return launch_tile<XF32, XP, EP, 2, 4>(a, st);
+  if (blocks(1, 4) >= kMinBlocks) return launch_tile<XF32, XP, EP, 1, 4>(a, st);
+  if (blocks(1, 2) >= kMinBlocks) return launch_tile<XF32, XP, EP, 1, 2>(a, st);
+  return launch_tile<XF32, XP, EP, 1, 1>(a, st);
+}
+
+}  // namespace
+
+int launch_rows(const RowsArgs& a, bool xf32, int xp, int ep, hipStream_t st) {
+  if (!a.w || !a.s || !a.x || !a.y || (ep == EP_RESID && !a.resid)) return Q4D_ERR_NULL;
+  if (a.M <= 0 || a.M > 16 * 65535 || a.N <= 0 || a.K <= 0 || a.K % kRwUnit) return Q4D_ERR_SHAPE;
+  if (!aligned(a.w, 16) || !aligned(a.s, 4) || !aligned(a.x, 16)) return Q4D_ERR_BAD_ADDR;
+  if (xf32 && ep == EP_RESID) return Q4D_ERR_DTYPE;
+  if (xf32 && xp == 2) return ep == EP_F16 ? launch_nt<true, 2, EP_F16>(a, st) : launch_nt<true, 2, EP_F32>(a, st);
+  if (xf32) return ep == EP_F16 ? launch_nt<true, 1, EP_F16>(a, st) : launch_nt<true, 1, EP_F32>(a, st);
+  switch (ep) {
+    case EP_F16: return launch_nt<false, 1, EP_F16>(a, st);
+    case EP_F32: return launch_nt<false, 1, EP_F32>(a, st);
+    case EP_RESID: return launch_nt<false, 1, EP_RESID>(a, st);
+    default: return Q4D_ERR_SHAPE;
+  }
+}
+
+}  // namespace q4d

@@ -1,0 +1,80 @@
+"""q4d_linear over several activation rows (the MFMA kernel of 4 rows and more) on the GPU
+vs the oracle: tile edges in both directions, every matrix width, every input and output type."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as o
+from gpu_helpers import linear, q4
+from llm_accelerator_amd import _lib
+from llm_accelerator_amd._lib import Q4D_F16, Q4D_F32
+
+pytestmark = pytest.mark.gpu
+
+ACC = 4e-6  # fp32 accumulation error relative to sum |w x|, the bar of the one-row GEMV
+
+
+@pytest.mark.parametrize("m,n,k,xdtype,ydtype,precision", [
+    (4, 2, 1024, torch.float32, Q4D_F32, 2),         # one tile, nearly empty
+    (16, 1024, 2048, torch.float32, Q4D_F32, 2),     # one row tile, one weight tile per block
+    (17, 1030, 1024, torch.float16, Q4D_F16, 1),     # ragged both ways, fp16 in and out
+    (33, 3072, 3072, torch.float32, Q4D_F32, 2),     # two weight tiles per block
+    (211, 1024, 3072, torch.float32, Q4D_F16, 2),    # four weight tiles per block
+    (300, 2050, 2048, torch.float16, Q4D_F32, 1),
+    (50, 96, 1024, torch.float32, Q4D_F32, 1),       # fp32 activations rounded to fp16
+])
+def test_linear_rows_vs_oracle(dev, m, n, k, xdtype, ydtype, precision):
+    rng = np.random.default_rng(m + n + k)
+    packed = rng.integers(0, 256, size=(n, k // 2), dtype=np.uint8)
+    scale = rng.integers(1, 3000, size=(n, k // 64)).astype(np.uint16)
+    x = rng.normal(size=(m, k)) * 10.0 ** rng.integers(-3, 3, size=(m, 1))  # small rows: denormal lo halves
+    xt = torch.from_numpy(x.astype(np.float32)).to(dev).to(xdtype)
+    lib = _lib.load()
+    _lib.check(lib.q4d_set_activation_precision(precision), "q4d_set_activation_precision")
+    try:
+        y = linear(q4(packed, scale, dev), xt, ydtype).double().cpu().numpy()
+    finally:
+        _lib.check(lib.q4d_set_activation_precision(2), "q4d_set_activation_precision")
+    W = o.dequantize_q4(packed, scale, dtype=np.float64)
+    x64 = xt.double().cpu().numpy()
+    ref, size = x64 @ W.T, np.abs(x64) @ np.abs(W).T
+    # hi + lo halves: 2^-22 of a value, and no finer than the fp16 denormal step 2^-25 of the
+    # lo half; one fp16 value: 2^-11, and no finer than 2^-25
+    lone = np.abs(W).sum(axis=1)[None, :] * 2.0 ** -25
+    xerr = 0.0 if xdtype == torch.float16 else size * (2.0 ** -22 if precision == 2 else 2.0 ** -11) + lone
+    out = np.abs(ref) * 2.0 ** -11 + 2.0 ** -25 if ydtype == Q4D_F16 else 0.0
+    finite = np.abs(ref) < 65000 if ydtype == Q4D_F16 else np.ones_like(ref, dtype=bool)
+    assert finite.mean() > 0.5
+    assert np.all((np.abs(y - ref) <= ACC * size + xerr + out)[finite])
+
+
+def test_linear_rows_one_bad_row_stays_alone(dev):
+    """A row holding an infinity or a NaN does not reach the other rows of its tile."""
+    rng = np.random.default_rng(3)
+    w = q4(rng.integers(0, 256, size=(64, 512), dtype=np.uint8), np.full((64, 16), 100, dtype=np.uint16), dev)
+    x = torch.randn(20, 1024, device=dev)
+    clean = linear(w, x)
+    x[5, 17], x[9, 1000] = float("inf"), float("nan")
+    y = linear(w, x)
+    keep = [i for i in range(20) if i not in (5, 9)]
+    assert torch.equal(y[keep], clean[keep])
+    assert not torch.isfinite(y[5]).any() and not torch.isfinite(y[9]).any()
+
+
+def test_linear_group_rows_equal_single_calls(dev):
+    """q4d_linear_group at 4 rows and more: each output equals its own q4d_linear call."""
+    from llm_accelerator_amd.model import current_stream
+    rng = np.random.default_rng(4)
+    ws = [q4(rng.integers(0, 256, size=(130, 512), dtype=np.uint8),
+             rng.integers(1, 3000, size=(130, 16)).astype(np.uint16), dev) for _ in range(3)]
+    xs = [torch.randn(18, 1024, device=dev) for _ in ws]
+    ys = [torch.full((18, 130), float("nan"), device=dev) for _ in ws]
+    descs = (_lib.Q4dMatrix * 3)(*[w.descriptor() for w in ws])
+    xp, yp = ((ctypes.c_void_p * 3)(*[t.data_ptr() for t in ts]) for ts in (xs, ys))
+    _lib.check(_lib.load().q4d_linear_group(descs, xp, Q4D_F32, yp, Q4D_F32, 18, 3, current_stream()),
+               "q4d_linear_group")
+    for w, x, y in zip(ws, xs, ys):
+        assert torch.equal(y, linear(w, x))
