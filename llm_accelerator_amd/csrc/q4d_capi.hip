@@ -612,6 +612,7 @@ int q4d_gemm(const q4d_matrix_t* w, const uint16_t* x, int32_t M, void* y, int32
   a.y = y;
   a.ldy = w->rows;
   a.resid = resid;
+  a.rows = 1;
   return launch_gemm(a, resid ? EP_RESID : (y_dtype == Q4D_F16 ? EP_F16 : EP_F32), false, as_stream(stream));
 }
 
@@ -657,7 +658,7 @@ int q4d_gemm_splitk(const q4d_matrix_t* w, const uint16_t* x, int32_t M, void* y
   a.part = part;
   a.part_cap = part_bytes / 4;
   a.ksplit = ksplit;
-  a.skinny = ksplit == 0;  // the library chooses: the skinny kernel for M <= 64
+  a.rows = a.skinny = ksplit == 0;  // the library chooses
   return launch_gemm(a, resid ? EP_RESID : (y_dtype == Q4D_F16 ? EP_F16 : EP_F32), false, as_stream(stream));
 }
 

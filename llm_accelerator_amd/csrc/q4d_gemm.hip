@@ -1131,6 +1131,21 @@ static int launch_gemm_bm(const GemmArgs& a, int ep, bool pair, hipStream_t st) 
   }
 }
 
+// Whether the rows kernel (q4d_rows.hip) runs: asked for, one matrix, and few enough outputs.
+// The tiled kernels' time there is their chain of K steps on too few blocks, whatever M is
+// (K = 1024 / 2048 / 3072: 12-15 / 22-24 / 31-34 us up to the sizes below); the rows kernel
+// splits K over the waves of a block: 64 rows of 3072 x 1024 12.6 -> 5.2 us, of 1024 x 3072
+// 32.7 -> 4.0, 512 rows 14.5 -> 11.9 and 33.8 -> 10.1, 1024 x 1024 x 3072 34.0 -> 18.2.  Both
+// grow with K, so they cross at a number of outputs: 3072 x 1024 between 512 and 768 rows,
+// 2048 x 1024 at 1024, 1024 x 3072 between 1024 and 2048.  Widths other than the projections'
+// take the kernel's general loop, which is slower: up to 64 rows.
+static bool rows_apply(const GemmArgs& a, int ep, bool pair) {
+  if (!a.rows || pair || a.nseg != 1 || (ep != EP_F16 && ep != EP_F32 && ep != EP_RESID)) return false;
+  if (a.ldy != a.N || a.K % 128 || !aligned(a.s[0], 4)) return false;
+  if (a.K != 1024 && a.K != 2048 && a.K != 3072) return a.M <= 64;
+  return (long long)a.M * a.N <= 1750000;
+}
+
 int launch_gemm(const GemmArgs& a, int ep, bool pair, hipStream_t st) {
   if (a.M <= 0 || a.K <= 0 || a.K % kGemmBK || a.N <= 0) return Q4D_ERR_SHAPE;
   if (a.nseg < 1 || a.nseg > 3) return Q4D_ERR_SHAPE;
@@ -1158,6 +1173,9 @@ int launch_gemm(const GemmArgs& a, int ep, bool pair, hipStream_t st) {
     return Q4D_ERR_NULL;
   }
   if (ep == EP_RESID && !a.resid) return Q4D_ERR_NULL;
+  if (rows_apply(a, ep, pair))
+    return launch_rows(RowsArgs{a.w[0], a.s[0], a.x, a.y, ep == EP_RESID ? a.resid : nullptr, a.M, a.N, a.K}, false, 0,
+                       ep, st);
   // large M (prefill): the pipelined kernel, 128-row tiles
   if (a.M > 64 && ep != EP_ARGMAX && pipe_steps(a, pair)) {
     if (pair) return ep == EP_SWIGLU ? launch_gemm_pipe<EP_SWIGLU, true>(a, st) : Q4D_ERR_SHAPE;

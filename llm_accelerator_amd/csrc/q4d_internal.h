@@ -364,6 +364,8 @@ struct GemmArgs {
   int skinny;
   int x_tiled;
   int y_tiled;
+  // rows: the kernel of q4d_rows.hip may run (its sums are grouped differently too)
+  int rows;
   int* ksplit_used;  // optional: receives the split launch_gemm ran (1: the epilogue was applied)
   // EP_ROPE (prefill q|k|v, no split): the 128 columns of an output tile are one
   // head, q heads then k heads then v heads; q rows go normed, roped and scaled to

@@ -33,13 +33,16 @@ constexpr int kRwUnit = 128;           // K columns per wave and step
 constexpr int kRwLd = kRwUnit + 16;    // LDS row stride in fp16: 288 B, conflict-free MFMA operand reads
 constexpr int kRwRed = 17;             // LDS row stride (floats) of the partial tiles
 
-// XF32: fp32 activations (else fp16).  XP: 2 = hi + lo halves, 1 = one fp16 value.  The block's
+// XF32: fp32 activations (else fp16).  XP: 2 = hi + lo halves, 1 = one fp16 value, 0 = one fp16
+// value and the weights rounded to fp16 as q4d_gemm states it (one rounding of code x scale,
+// so no scale is applied to the sums).  The block's
 // tile is 16 MT activation rows x 16 NT weight rows.  UPW > 0: every wave has UPW units and
 // issues all their loads at entry; 0: any number, the next unit's loads in flight.
 template <bool XF32, int XP, int EP, int MT, int NT, int NW, int UPW>
 __global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
-  static_assert(XF32 || XP == 1, "fp16 activations are one value");
-  constexpr int kX = NW * XP * 16 * MT * kRwLd * 2, kR = NW * MT * NT * 16 * kRwRed * 4;
+  static_assert(XF32 ? XP != 0 : XP != 2, "fp16 activations are one value");
+  constexpr int kH = XP == 2 ? 2 : 1;
+  constexpr int kX = NW * kH * 16 * MT * kRwLd * 2, kR = NW * MT * NT * 16 * kRwRed * 4;
   __shared__ __attribute__((aligned(16))) char lds[kX > kR ? kX : kR];
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -47,7 +50,7 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
   const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
   const int nu = a.K / kRwUnit;
   const int u0 = w * nu / NW, u1 = (w + 1) * nu / NW;
-  _Float16* xs = reinterpret_cast<_Float16*>(lds) + (size_t)w * XP * 16 * MT * kRwLd;
+  _Float16* xs = reinterpret_cast<_Float16*>(lds) + (size_t)w * kH * 16 * MT * kRwLd;
 
   // rows past the end read the last one; their results are not stored
   // (32-bit offsets from the block's first rows: one address register per load)
@@ -122,6 +125,14 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
     for (int j = 0; j < NT; ++j) rows_transpose4(d4[j]);
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
+      h2 sh[NT];
+      if constexpr (XP == 0) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          const _Float16 f = (_Float16)scale_q2_14(g ? sc[j] >> 16 : sc[j] & 0xFFFFu);
+          sh[j] = make_h2(f, f);
+        }
+      }
       f32x4 p[MT][NT];
 #pragma unroll
       for (int i = 0; i < MT; ++i)
@@ -138,6 +149,13 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
         }
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
+          if constexpr (XP == 0) {
+            const h8 q = __builtin_bit_cast(h8, dequant8(d4[j][s], sh[j]));
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+              tot[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[i], q, tot[i][j], 0, 0, 0);
+            continue;
+          }
           const h8 q = __builtin_bit_cast(h8, codes8(d4[j][s]));
 #pragma unroll
           for (int i = 0; i < MT; ++i) {
@@ -146,6 +164,7 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
           }
         }
       }
+      if constexpr (XP == 0) continue;
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         const float f = scale_q2_14(g ? sc[j] >> 16 : sc[j] & 0xFFFFu);
@@ -200,7 +219,7 @@ int launch_tile(const RowsArgs& a, hipStream_t st) {
   // Every unit of a wave in flight where K is one of the projections' widths and the
   // registers hold them (211 x 1024 x 3072, hi + lo: 9.5 us, 11.5 with the next unit only);
   // K = 3072 on one-tile blocks: 12 waves of two units (4 rows: 5.1 us, 5.5 with 8 of three).
-  constexpr bool kSmall = MT == 1 && NT == 1, kDeep = XP == 1 || MT * NT <= 4;
+  constexpr bool kSmall = MT == 1 && NT == 1, kDeep = XP < 2 || MT * NT <= 4;
   const int nu = a.K / kRwUnit;
   if (nu == 8)
     go(rows_kernel<XF32, XP, EP, MT, NT, 8, 1>, 8);
@@ -235,14 +254,16 @@ int launch_rows(const RowsArgs& a, bool xf32, int xp, int ep, hipStream_t st) {
   if (!a.w || !a.s || !a.x || !a.y || (ep == EP_RESID && !a.resid)) return Q4D_ERR_NULL;
   if (a.M <= 0 || a.M > 16 * 65535 || a.N <= 0 || a.K <= 0 || a.K % kRwUnit) return Q4D_ERR_SHAPE;
   if (!aligned(a.w, 16) || !aligned(a.s, 4) || !aligned(a.x, 16)) return Q4D_ERR_BAD_ADDR;
-  if (xf32 && ep == EP_RESID) return Q4D_ERR_DTYPE;
+  if (ep != EP_F16 && ep != EP_F32 && ep != EP_RESID) return Q4D_ERR_SHAPE;
+  if (xf32 ? xp < 1 || xp > 2 : xp < 0 || xp > 1) return Q4D_ERR_DTYPE;
+  if (ep == EP_RESID && (xf32 || xp)) return Q4D_ERR_DTYPE;
   if (xf32 && xp == 2) return ep == EP_F16 ? launch_nt<true, 2, EP_F16>(a, st) : launch_nt<true, 2, EP_F32>(a, st);
   if (xf32) return ep == EP_F16 ? launch_nt<true, 1, EP_F16>(a, st) : launch_nt<true, 1, EP_F32>(a, st);
+  if (xp == 1) return ep == EP_F16 ? launch_nt<false, 1, EP_F16>(a, st) : launch_nt<false, 1, EP_F32>(a, st);
   switch (ep) {
-    case EP_F16: return launch_nt<false, 1, EP_F16>(a, st);
-    case EP_F32: return launch_nt<false, 1, EP_F32>(a, st);
-    case EP_RESID: return launch_nt<false, 1, EP_RESID>(a, st);
-    default: return Q4D_ERR_SHAPE;
+    case EP_F16: return launch_nt<false, 0, EP_F16>(a, st);
+    case EP_F32: return launch_nt<false, 0, EP_F32>(a, st);
+    default: return launch_nt<false, 0, EP_RESID>(a, st);
   }
 }
 

@@ -78,3 +78,26 @@ def test_linear_group_rows_equal_single_calls(dev):
                "q4d_linear_group")
     for w, x, y in zip(ws, xs, ys):
         assert torch.equal(y, linear(w, x))
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 128, 1024), (33, 1024, 3072), (64, 384, 2048), (100, 3072, 1024), (500, 3072, 1024),
+                                   (401, 1024, 3072), (64, 128, 1152)])
+def test_gemm_few_outputs_vs_fp16_operands(dev, m, n, k):
+    """q4d_gemm where it takes the rows kernel: the product of the same fp16 operands (weights
+    rounded once), every tile size and the general K loop (1152 columns)."""
+    from llm_accelerator_amd.model import current_stream
+    rng = np.random.default_rng(m + n + k)
+    packed = rng.integers(0, 256, size=(n, k // 2), dtype=np.uint8)
+    scale = rng.integers(1, 1500, size=(n, k // 64)).astype(np.uint16)
+    w = q4(packed, scale, dev)
+    x = torch.from_numpy(rng.normal(size=(m, k)).astype(np.float16)).to(dev)
+    resid = torch.from_numpy(rng.normal(size=(m, n)).astype(np.float32)).to(dev)
+    y = torch.full((m, n), float("nan"), device=dev)
+    desc = w.descriptor()
+    _lib.check(_lib.load().q4d_gemm(ctypes.byref(desc), x.data_ptr(), m, y.data_ptr(), Q4D_F32, resid.data_ptr(),
+                                    current_stream()), "q4d_gemm")
+    q = o.unpack_signed_int4(packed, k).astype(np.float16)
+    w16 = (q * np.repeat((scale / 16384.0).astype(np.float16), 64, axis=1)).astype(np.float64)
+    x64 = x.double().cpu().numpy()
+    bound = 2.0 ** -16 * (np.abs(x64) @ np.abs(w16).T) + 2.0 ** -22
+    assert np.all(np.abs(y.double().cpu().numpy() - resid.double().cpu().numpy() - x64 @ w16.T) <= bound)
