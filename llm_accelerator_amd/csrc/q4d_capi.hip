@@ -956,6 +956,7 @@ int q4d_prefill(const q4d_model_t* model, const int32_t* tokens, int32_t n_token
     g.N = g.seg_end[2]; g.K = H; g.M = n;
     g.x = xh;
     g.rope = pa;
+    g.chain = 1;
     if ((rc = launch_gemm(g, EP_ROPE, false, st))) return rc;
 
     // causal GQA attention over positions [0, start_pos + n)
@@ -967,6 +968,7 @@ int q4d_prefill(const q4d_model_t* model, const int32_t* tokens, int32_t n_token
     g.seg_end[0] = H; g.nseg = 1;
     g.N = H; g.K = qh * d; g.M = n;
     g.x = ws_ptr<uint16_t>(ws, P.attn); g.y = hidden; g.ldy = H; g.resid = hidden;
+    g.chain = 1;
     g.part = ws_ptr<float>(ws, P.part); g.part_cap = (size_t)kPrefillSplit * n * H; g.ksplit = kPrefillSplit;
     g.defer_reduce = 1;  // split sums + residual + post-attention RMSNorm in one pass
     if ((rc = launch_gemm(g, EP_RESID, false, st))) return rc;
@@ -979,12 +981,14 @@ int q4d_prefill(const q4d_model_t* model, const int32_t* tokens, int32_t n_token
     g.seg_end[0] = I; g.seg_end[1] = 2 * I; g.nseg = 2;
     g.N = I; g.K = H; g.M = n;
     g.x = xh; g.y = act; g.ldy = I;
+    g.chain = 1;
     if ((rc = launch_gemm(g, EP_SWIGLU, true, st))) return rc;
     memset(&g, 0, sizeof(g));
     g.w[0] = L.down_proj.w; g.s[0] = L.down_proj.s;
     g.seg_end[0] = H; g.nseg = 1;
     g.N = H; g.K = I; g.M = n;
     g.x = act; g.y = hidden; g.ldy = H; g.resid = hidden;
+    g.chain = 1;
     g.part = ws_ptr<float>(ws, P.part); g.part_cap = (size_t)kPrefillSplit * n * H; g.ksplit = kPrefillSplit;
     if (l + 1 < model->num_layers) {  // split sums + residual + the next layer's input RMSNorm
       g.defer_reduce = 1;

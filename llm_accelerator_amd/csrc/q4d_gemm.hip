@@ -201,11 +201,7 @@ __device__ __forceinline__ void rope_epilogue(const GemmArgs& a, const f32x4 (&a
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      float v = acc[i][0][r] * acc[i][0][r];
-      v = fmaf(acc[i][1][r], acc[i][1][r], v);
-      v = fmaf(acc[i][2][r], acc[i][2][r], v);
-      v = fmaf(acc[i][3][r], acc[i][3][r], v);
-      v = row16_sum(v);
+      const float v = rope_half_ss(acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]);
       if (cl == 0) ssx[wn * BM + wm + 16 * i + rq + r] = v;
     }
   __syncthreads();
@@ -215,19 +211,16 @@ __device__ __forceinline__ void rope_epilogue(const GemmArgs& a, const f32x4 (&a
     for (int r = 0; r < 4; ++r) {
       const int row = wm + 16 * i + rq + r, tok = m0 + row;
       if (tok >= a.M) continue;
-      const float ss = ssx[row] + ssx[BM + row];
-      const float inv = 1.0f / sqrtf(ss / (float)kGemmBN + R.eps);
+      const float inv = rope_inv(ssx[row] + ssx[BM + row], R.eps);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int d = 32 * wn + 16 * j + cl;
-        const float n0 = (acc[i][j][r] * inv) * g0[j], n1 = (acc[i][j + 2][r] * inv) * g1[j];
-        // rotate_half: dim d < 64 takes -x[d + 64], dim d + 64 takes x[d]
-        const float r0 = n0 * cs[i][r][j] - n1 * sn[i][r][j];
-        const float r1 = n1 * cs[i][r][j] + n0 * sn[i][r][j];
+        float r0 = acc[i][j][r], r1 = acc[i][j + 2][r];
+        rope_pair(r0, r1, inv, g0[j], g1[j], cs[i][r][j], sn[i][r][j]);
         if (isq) {
           _Float16* dst = R.q16 + ((size_t)h * R.n + tok) * kGemmBN;
-          dst[d] = (_Float16)(r0 * R.qscale);
-          dst[d + 64] = (_Float16)(r1 * R.qscale);
+          dst[d] = rope_q_lo(r0, R.qscale);
+          dst[d + 64] = rope_q_hi(r1, R.qscale);
         } else {
           uint16_t* dst = R.kcache + ((size_t)(h - R.qh) * R.max_ctx + R.p0 + tok) * kGemmBN;
           dst[d] = __builtin_bit_cast(uint16_t, (_Float16)r0);
@@ -348,8 +341,7 @@ __global__ __launch_bounds__(NW * 64) void q4_gemm_kernel(const GemmArgs a) {
           const int m = m0 + wm + 16 * i + rq + r;
           if (m < a.M) {
             const float g = acc[i][j][r], u = acc[i][j + 2][r];
-            const float act = (g / (1.0f + expf(-g))) * u;
-            static_cast<_Float16*>(a.y)[(size_t)m * a.ldy + n] = (_Float16)act;
+            static_cast<_Float16*>(a.y)[(size_t)m * a.ldy + n] = swiglu(g, u);
           }
         }
       }
@@ -721,8 +713,7 @@ __global__ __launch_bounds__(512) void q4_gemm_pipe_kernel(const GemmArgs a) {
           const int m = m0 + wm + 16 * i + rq + r;
           if (m < a.M) {
             const float g = acc[i][j][r], u = acc[i][j + 2][r];
-            const float act = (g / (1.0f + expf(-g))) * u;
-            static_cast<_Float16*>(a.y)[(size_t)m * a.ldy + n] = (_Float16)act;
+            static_cast<_Float16*>(a.y)[(size_t)m * a.ldy + n] = swiglu(g, u);
           }
         }
       }
@@ -1176,6 +1167,14 @@ int launch_gemm(const GemmArgs& a, int ep, bool pair, hipStream_t st) {
   if (rows_apply(a, ep, pair))
     return launch_rows(RowsArgs{a.w[0], a.s[0], a.x, a.y, ep == EP_RESID ? a.resid : nullptr, a.M, a.N, a.K}, false, 0,
                        ep, st);
+  if (a.chain && chain_applies(a, ep, pair)) {
+    if (a.ksplit_used) *a.ksplit_used = a.ksplit > 1 ? a.ksplit : 1;
+    const int rc = launch_chain(a, ep, pair, st);
+    if (rc || a.ksplit <= 1 || a.defer_reduce) return rc;
+    const int n4 = a.M * (a.N / 4);
+    hipLaunchKernelGGL((splitk_reduce_kernel<EP_RESID, false>), dim3((n4 + 255) / 256), dim3(256), 0, st, a, a.ksplit);
+    return check_launch();
+  }
   // large M (prefill): the pipelined kernel, 128-row tiles
   if (a.M > 64 && ep != EP_ARGMAX && pipe_steps(a, pair)) {
     if (pair) return ep == EP_SWIGLU ? launch_gemm_pipe<EP_SWIGLU, true>(a, st) : Q4D_ERR_SHAPE;

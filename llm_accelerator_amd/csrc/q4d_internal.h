@@ -366,6 +366,8 @@ struct GemmArgs {
   int y_tiled;
   // rows: the kernel of q4d_rows.hip may run (its sums are grouped differently too)
   int rows;
+  // chain: the kernel of q4d_chain.hip may run (prefill; the same sums bit for bit)
+  int chain;
   int* ksplit_used;  // optional: receives the split launch_gemm ran (1: the epilogue was applied)
   // EP_ROPE (prefill q|k|v, no split): the 128 columns of an output tile are one
   // head, q heads then k heads then v heads; q rows go normed, roped and scaled to
@@ -373,6 +375,10 @@ struct GemmArgs {
   // at positions rope.p0 + m.  y is not written.
   PrefillArgs rope;
 };
+// The prefill GEMMs of short prompts (q4d_chain.hip): EP_ROPE and EP_SWIGLU without a split,
+// EP_RESID with a.ksplit splits into a.part (raw partial tiles; the reduction is the caller's).
+bool chain_applies(const GemmArgs& a, int ep, bool pair);
+int launch_chain(const GemmArgs& a, int ep, bool pair, hipStream_t st);
 constexpr int kGemmMaxSplit = 16;
 // Compute units of the current device (cached per process; 256 on MI355X).
 int device_cus();

@@ -57,4 +57,40 @@ __device__ __forceinline__ void rows_transpose4(uint32_t (&d)[4]) {
   d[3] = f[1];
 }
 
+// ---- arithmetic the prefill GEMM epilogues share ------------------------------------
+// A prompt in chunks gives the same bits as one call whichever kernel a chunk's size picks,
+// so the roundings are spelt out: sums as explicit fused multiply-adds, and a product that
+// goes to fp16 either rounded once (mul_f16) or pinned in fp32 first.  Left to itself the
+// compiler may choose differently in each kernel.
+__device__ __forceinline__ float pin_f32(float v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+// a * b rounded once to fp16.
+__device__ __forceinline__ _Float16 mul_f16(float a, float b) {
+  uint32_t d;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(d) : "v"(a), "v"(b));
+  return __builtin_bit_cast(_Float16, (uint16_t)d);
+}
+
+__device__ __forceinline__ _Float16 swiglu(float g, float u) { return mul_f16(g / (1.0f + expf(-g)), u); }
+
+// One head's row in the hands of two 16-lane rows: lane cl of half wn holds x[j] = dims
+// 32 wn + 16 j + cl and x[j + 2] = their rotate-half partners + 64 (j = 0, 1).
+// This half's part of the sum of squares (the same in its 16 lanes):
+__device__ __forceinline__ float rope_half_ss(float x0, float x1, float x2, float x3) {
+  return row16_sum(fmaf(x3, x3, fmaf(x2, x2, fmaf(x1, x1, x0 * x0))));
+}
+__device__ __forceinline__ float rope_inv(float ss, float eps) { return 1.0f / sqrtf(fmaf(ss, 1.0f / 128.0f, eps)); }
+// RMSNorm scale, gamma and rotation of dim d (a) and d + 64 (b), in place:
+__device__ __forceinline__ void rope_pair(float& a, float& b, float inv, float ga, float gb, float c, float s) {
+  const float n0 = (a * inv) * ga, n1 = (b * inv) * gb;
+  a = fmaf(n0, c, -pin_f32(n1 * s));
+  b = fmaf(n0, s, pin_f32(n1 * c));
+}
+// q leaves with the softmax scale folded in: dim d rounded once, dim d + 64 after an fp32
+// product.
+__device__ __forceinline__ _Float16 rope_q_lo(float v, float qscale) { return mul_f16(v, qscale); }
+__device__ __forceinline__ _Float16 rope_q_hi(float v, float qscale) { return (_Float16)pin_f32(v * qscale); }
+
 }  // namespace q4d
