@@ -15,8 +15,10 @@
 // the raw partial tile of a K split.
 //
 // What bounds it: the launch, one memory round trip and the unpacking VALU work of the two
-// waves on each SIMD (75 tokens, kernel times: q|k|v 8.7 us, was 17.0; gate / up 8.7, 15.4;
-// o_proj 6.6, 16.0; down 6.6, 21.9; the 28 layers and LM head 2380 -> 1224 us).
+// waves on each SIMD (75 tokens, kernel times: q|k|v 8.0 us, was 17.0; gate / up 7.7, 15.4;
+// o_proj and down 5.7 on average, 16.0 and 21.9; the 28 layers and LM head 2385 -> 1131 us).
+#include <type_traits>
+
 #include "q4d_internal.h"
 #include "q4d_mfma_dev.h"
 
@@ -80,29 +82,37 @@ __global__ __launch_bounds__(NW * 64) void q4_chain_kernel(const GemmArgs a) {
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
     const int q = t + NT * i;
-    *reinterpret_cast<u32x4*>(xs + (q / CPR) * LD + (q % CPR) * 8) = x[i];
+    *reinterpret_cast<u32x4*>(xs + (q / CPR) * LD + (q % CPR) * 8) = to_pairs(x[i]);
   }
   block_sync_lds();
 
   f32x4 acc[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const auto units = [&](auto wide) {
 #pragma unroll
-  for (int u = 0; u < NU; ++u) {
-    uint32_t d[4] = {c[u][0], c[u][1], c[u][2], c[u][3]};
-    rows_transpose4(d);
-    const _Float16 slo = (_Float16)scale_q2_14(sc[u] & 0xFFFFu), shi = (_Float16)scale_q2_14(sc[u] >> 16);
+    for (int u = 0; u < NU; ++u) {
+      uint32_t d[4] = {c[u][0], c[u][1], c[u][2], c[u][3]};
+      rows_transpose4(d);
+      const W16Scale lo = w16_scale(sc[u] & 0xFFFFu), hi = w16_scale(sc[u] >> 16);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const _Float16 f = s < 2 ? slo : shi;
-      const h8 q = __builtin_bit_cast(h8, dequant8(d[s], make_h2(f, f)));
+      for (int s = 0; s < 4; ++s) {
+        const h8 q = __builtin_bit_cast(h8, dequant8_pairs<decltype(wide)::value>(d[s], s < 2 ? lo : hi));
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const h8 xv = *reinterpret_cast<const h8*>(xs + (16 * i + nl) * LD + kChUnit * u + 32 * s + 8 * G);
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, q, acc[i], 0, 0, 0);
+        for (int i = 0; i < MT; ++i) {
+          const h8 xv = *reinterpret_cast<const h8*>(xs + (16 * i + nl) * LD + kChUnit * u + 32 * s + 8 * G);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, q, acc[i], 0, 0, 0);
+        }
       }
     }
-  }
+  };
+  uint32_t most = 0;
+#pragma unroll
+  for (int u = 0; u < NU; ++u) most = max(most, max(sc[u] & 0xFFFFu, sc[u] >> 16));
+  if (scale_wide(most))
+    units(std::true_type{});
+  else
+    units(std::false_type{});
 
   // lane holds token rows 16 i + 4G + r of column 16 w + l % 16
   __syncthreads();

@@ -5,11 +5,8 @@
 // When many activation rows share each weight (prefill, batched decode), the
 // work becomes a dense contraction: each 128(N) x 64(K) Q4 tile (one scale
 // group per row) is dequantised once per block into LDS as fp16 and read by
-// every MFMA of the block.  Dequantisation uses packed fp16: after
-// v = w ^ 0x88888888 the nibble u = q + 8 placed in the low byte of an fp16
-// with exponent bits 0x6400 reads 1024 + u, so (0x6400|u) - 1032 = q exactly,
-// and q * scale is one correctly rounded fp16 multiply (the scale code is an
-// exact fp16 below 2048, i.e. scale < 0.125).
+// every MFMA of the block.  Dequantisation (q4d_mfma_dev.h) is one packed fp16 fma per pair,
+// with the rounding of a fp16 product q * scale.
 //
 // Block tile 128 (M, BM = 128) or 64 (BM = 64) x 128 (N) x 64 (K), 256 threads
 // = 2 x 2 waves; each wave owns (BM/2) x 64 of the output as 16x16 tiles of
@@ -44,14 +41,18 @@ constexpr int kGemmBK = 64;
 constexpr int kGemmPad = 16;
 constexpr int kGemmLds = kGemmBK + kGemmPad;
 
-// Dequantise 32 consecutive int4 (one 16-byte chunk) times `scale` to fp16,
-// in column order.
-__device__ __forceinline__ void dequant32(const u32x4 w, h2 scale2, uint32_t (&out)[16]) {
+// NW words of consecutive int4 times the scale of `code` to fp16, in column order.  FAST: the
+// one-fma conversion where no lane of the wave has a scale code past it; else the general one
+// without a branch.
+template <bool FAST, int NW>
+__device__ __forceinline__ void dequant_words(const uint32_t (&w)[NW], uint32_t code, u32x4 (&out)[NW]) {
+  const W16Scale f = w16_scale(code);
+  if (!FAST || scale_wide(code)) {
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const u32x4 o = dequant8(w[m], scale2);
+    for (int m = 0; m < NW; ++m) out[m] = dequant8<true>(w[m], f);
+  } else {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) out[4 * m + p] = o[p];
+    for (int m = 0; m < NW; ++m) out[m] = dequant8<false>(w[m], f);
   }
 }
 
@@ -124,7 +125,7 @@ __device__ __forceinline__ void gemm_load(const GemmArgs& a, const SegPtrs& P, i
   L.s = sb[(size_t)grow * (a.K / 64) + k0 / 64];
 }
 
-template <int BM, int NT>
+template <int BM, int NT, bool FAST>
 __device__ __forceinline__ void gemm_store_lds(_Float16 (*As)[kGemmLds], _Float16 (*Bs)[kGemmLds], int t,
                                                const GemmTileLoad& L) {
 #pragma unroll
@@ -134,12 +135,12 @@ __device__ __forceinline__ void gemm_store_lds(_Float16 (*As)[kGemmLds], _Float1
   }
   if (t >= 256) return;
   const int r = t >> 1, half = t & 1;
-  const _Float16 sc = (_Float16)((float)L.s * (1.0f / 16384.0f));
-  uint32_t out[16];
-  dequant32(L.w, make_h2(sc, sc), out);
+  const uint32_t cw[4] = {L.w[0], L.w[1], L.w[2], L.w[3]};
+  u32x4 out[4];
+  dequant_words<FAST>(cw, L.s, out);
   u32x4* dst = reinterpret_cast<u32x4*>(&Bs[r][half * 32]);
 #pragma unroll
-  for (int q = 0; q < 4; ++q) dst[q] = u32x4{out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]};
+  for (int q = 0; q < 4; ++q) dst[q] = out[q];
 }
 
 // ---- q|k|v epilogue of prefill (EP_ROPE) -------------------------------------------
@@ -281,10 +282,13 @@ __global__ __launch_bounds__(NW * 64) void q4_gemm_kernel(const GemmArgs a) {
     brow[j] = PAIR || EP == EP_ROPE ? ((j < 2) ? (32 * wn + 16 * j) : (64 + 32 * wn + 16 * (j - 2)))
                                     : (64 * wn + 16 * j);
 
+  // (2048 tokens: gate / up 42.2 -> 41.5 us, q|k|v 30.3 -> 29.3; the plain epilogues lose:
+  // 2000 x 3072 x 1024 23.1 -> 23.4)
+  constexpr bool kFast = EP == EP_SWIGLU || EP == EP_ROPE;
   const SegPtrs P = seg_ptrs(a);
   GemmTileLoad L;
   gemm_load<BM, PAIR, NT>(a, P, m0, nblk, k_begin * kGemmBK, t, L);
-  gemm_store_lds<BM, NT>(As[0], Bs[0], t, L);
+  gemm_store_lds<BM, NT, kFast>(As[0], Bs[0], t, L);
   __syncthreads();
 
   for (int ks = 0; ks < nk; ++ks) {
@@ -303,7 +307,7 @@ __global__ __launch_bounds__(NW * 64) void q4_gemm_kernel(const GemmArgs a) {
         for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[j], acc[i][j], 0, 0, 0);
       }
     }
-    if (ks + 1 < nk) gemm_store_lds<BM, NT>(As[buf ^ 1], Bs[buf ^ 1], t, L);
+    if (ks + 1 < nk) gemm_store_lds<BM, NT, kFast>(As[buf ^ 1], Bs[buf ^ 1], t, L);
     __syncthreads();
   }
 
@@ -436,24 +440,6 @@ __global__ __launch_bounds__(NW * 64) void q4_gemm_kernel(const GemmArgs a) {
 // the same number of loads per step and the waits are constants.
 constexpr int kPipeMaxGroups = 48;  // K <= 3072: Q2.14 scales of the block's rows, all K steps
 
-// 16 consecutive int4 (two words) times `scale` to fp16, in column order.
-__device__ __forceinline__ void dequant16(uint32_t w0, uint32_t w1, h2 scale2, uint32_t (&out)[8]) {
-  const h2 bias = make_h2((_Float16)1032.0f, (_Float16)1032.0f);
-#pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    const uint32_t v = (m ? w1 : w0) ^ 0x88888888u;
-    const uint32_t lo = v & 0x0F0F0F0Fu;
-    const uint32_t hi = (v >> 4) & 0x0F0F0F0Fu;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const uint32_t sel = (uint32_t)(p) | (0x0Cu << 8) | ((uint32_t)(4 + p) << 16) | (0x0Cu << 24);
-      const uint32_t pr = __builtin_amdgcn_perm(hi, lo, sel) | 0x64006400u;
-      const h2 q = __builtin_bit_cast(h2, pr) - bias;
-      out[4 * m + p] = __builtin_bit_cast(uint32_t, q * scale2);
-    }
-  }
-}
-
 // Row r (< 128) of the block's B tile: its segment's code / scale pointers and row.
 template <bool PAIR>
 __device__ __forceinline__ void pipe_brow(const SegPtrs& P, int nblk, int r, const uint8_t*& wb, const uint16_t*& sb,
@@ -550,12 +536,12 @@ template <int S, int B>
 __device__ __forceinline__ void pipe_dequant(const PipeCtx& c, int j) {
   const int r = c.t >> 2, q = c.t & 3;
   const u32x2 raw = *reinterpret_cast<const u32x2*>(&pipe_w<S>()[r][8 * q]);
-  const _Float16 sc = (_Float16)((float)g_psc[r][c.k_begin + j] * (1.0f / 16384.0f));
-  uint32_t out[8];
-  dequant16(raw[0], raw[1], make_h2(sc, sc), out);
+  const uint32_t cw[2] = {raw[0], raw[1]};
+  u32x4 out[2];
+  dequant_words<false>(cw, g_psc[r][c.k_begin + j], out);  // (with the branch: 1024 x 3072, 2000 rows 34.8 -> 38.0 us)
   u32x4* dst = reinterpret_cast<u32x4*>(&pipe_b<B>()[r][16 * q]);
-  dst[0] = u32x4{out[0], out[1], out[2], out[3]};
-  dst[1] = u32x4{out[4], out[5], out[6], out[7]};
+  dst[0] = out[0];
+  dst[1] = out[1];
 }
 
 // MFMAs of one K step: X from stage S, B from tile B.
@@ -816,15 +802,23 @@ __global__ __launch_bounds__(kSkMaxWaves * 64) void q4_skinny_kernel(const GemmA
 
   uint32_t d[4] = {wc[0], wc[1], wc[2], wc[3]};
   rows_transpose4(d);
-  const _Float16 slo = (_Float16)((float)(sc2 & 0xFFFFu) * (1.0f / 16384.0f));
-  const _Float16 shi = (_Float16)((float)(sc2 >> 16) * (1.0f / 16384.0f));
+  u32x4 wf[4];
+  {
+    const uint32_t lo[2] = {d[0], d[1]}, hi[2] = {d[2], d[3]};
+    u32x4 o[2];
+    dequant_words<true>(lo, sc2 & 0xFFFFu, o);
+    wf[0] = o[0];
+    wf[1] = o[1];
+    dequant_words<true>(hi, sc2 >> 16, o);
+    wf[2] = o[0];
+    wf[3] = o[1];
+  }
   f32x4 acc[4];
 #pragma unroll
   for (int ct = 0; ct < 4; ++ct) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
-    const _Float16 sc = s < 2 ? slo : shi;
-    const h8 af = __builtin_bit_cast(h8, dequant8(d[s], make_h2(sc, sc)));
+    const h8 af = __builtin_bit_cast(h8, wf[s]);
 #pragma unroll
     for (int ct = 0; ct < 4; ++ct)
       acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, __builtin_bit_cast(h8, xf[ct][s]), acc[ct], 0, 0, 0);

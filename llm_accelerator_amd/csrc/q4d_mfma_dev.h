@@ -7,36 +7,108 @@ namespace q4d {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
-// 8 consecutive int4 (one 32-bit word, low nibble first) as fp16 integers, in column
-// order: word p of the result holds columns 2p, 2p + 1.  (0x6400 | u) is 1024 + u, so
-// subtracting 1032 gives q = u - 8 exactly.
-__device__ __forceinline__ u32x4 codes8(uint32_t w) {
+// ---- int4 -> fp16 -----------------------------------------------------------------------
+// A 32-bit word holds columns 0..7, low nibble first, as two's complement int4.  A nibble
+// moved to bits 6..9 of an fp16 with its top bit flipped is the denormal u 2^-18, u = q + 8,
+// exactly linear in u; one packed fma per pair then gives
+//     (u 2^-18) (s 2^18) - 8 s = q s
+// rounded once, the same value as the fp16 product of q and s.  s 2^18 (the Q2.14 code times
+// 16) is a finite fp16 up to code 4094; larger codes (scale 0.25 and more) go through the
+// integers (codes_wide).  Shift + bit operation + fma per pair: 12 VALU instructions per
+// word in pair order, 16 in column order, against 20 through 0x6400 | u, subtract, multiply.
+constexpr uint32_t kScaleFastMax = 4094;
+
+struct W16Scale {
+  h2 mul, add;  // s 2^18 and -8 s, s = the fp16 scale
+  h2 s;
+};
+__device__ __forceinline__ W16Scale w16_scale(uint32_t code) {
+  const _Float16 m = (_Float16)((float)code * 16.0f), b = (_Float16)((float)code * (-8.0f / 16384.0f));
+  const _Float16 s = (_Float16)((float)code * (1.0f / 16384.0f));
+  return {make_h2(m, m), make_h2(b, b), make_h2(s, s)};
+}
+// Nibbles at bits 6..9 and 22..25, top bits flipped.
+__device__ __forceinline__ uint32_t nib_pair(uint32_t x) { return (x & 0x03C003C0u) ^ 0x02000200u; }
+
+// Whether any lane of the wave holds a scale code past the fast form's range.
+__device__ __forceinline__ bool scale_wide(uint32_t code) { return __builtin_amdgcn_ballot_w64(code > kScaleFastMax); }
+
+// fp16 integers of a word in pair order (word p = columns p, p + 4): (0x6400 | u) - 1032.
+__device__ __forceinline__ u32x4 codes_wide(uint32_t w) {
   const h2 bias = make_h2((_Float16)1032.0f, (_Float16)1032.0f);
   const uint32_t v = w ^ 0x88888888u;
-  const uint32_t lo = v & 0x0F0F0F0Fu;         // nibbles 0, 2, 4, 6 in bytes 0..3
-  const uint32_t hi = (v >> 4) & 0x0F0F0F0Fu;  // nibbles 1, 3, 5, 7
   u32x4 out;
 #pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    // fp16 pair (nibble 2p, nibble 2p+1): low byte of each half from lo / hi byte p
-    const uint32_t sel = (uint32_t)(p) | (0x0Cu << 8) | ((uint32_t)(4 + p) << 16) | (0x0Cu << 24);
-    const uint32_t pr = __builtin_amdgcn_perm(hi, lo, sel) | 0x64006400u;
-    out[p] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, pr) - bias);
+  for (int p = 0; p < 4; ++p)
+    out[p] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, ((v >> (4 * p)) & 0x000F000Fu) | 0x64006400u) - bias);
+  return out;
+}
+
+// q x scale in pair order: word p = columns p, p + 4 (an MFMA does not depend on the order of
+// the eight k values of a lane, as long as both operands share it).
+template <bool WIDE>
+__device__ __forceinline__ u32x4 dequant8_pairs(uint32_t w, const W16Scale& f) {
+  u32x4 out;
+  if constexpr (WIDE) {
+    const u32x4 q = codes_wide(w);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const uint32_t qp = q[p];
+      out[p] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, qp) * f.s);
+    }
+  } else {
+    const uint32_t x[4] = {w << 6, w << 2, w >> 2, w >> 6};
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      out[p] = __builtin_bit_cast(
+          uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, nib_pair(x[p])), f.mul, f.add));
   }
   return out;
 }
 
-// The same times `scale`: one correctly rounded fp16 multiply per element (the scale code
-// is an exact fp16 below 2048, i.e. scale < 0.125).
-__device__ __forceinline__ u32x4 dequant8(uint32_t w, h2 scale2) {
-  const u32x4 q = codes8(w);
+// q / 8 exactly, in pair order.
+__device__ __forceinline__ u32x4 codes8_pairs(uint32_t w) {
+  const h2 mul = make_h2((_Float16)32768.0f, (_Float16)32768.0f), add = make_h2((_Float16)-1.0f, (_Float16)-1.0f);
+  const uint32_t x[4] = {w << 6, w << 2, w >> 2, w >> 6};
   u32x4 out;
 #pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    const uint32_t qp = q[p];
-    out[p] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, qp) * scale2);
+  for (int p = 0; p < 4; ++p)
+    out[p] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, nib_pair(x[p])), mul, add));
+  return out;
+}
+
+// q x scale in column order: word p = columns 2p, 2p + 1.
+template <bool WIDE>
+__device__ __forceinline__ u32x4 dequant8(uint32_t w, const W16Scale& f) {
+  u32x4 out;
+  if constexpr (WIDE) {
+    const h2 bias = make_h2((_Float16)1032.0f, (_Float16)1032.0f);
+    const uint32_t v = w ^ 0x88888888u;
+    const uint32_t lo = v & 0x0F0F0F0Fu;         // nibbles 0, 2, 4, 6 in bytes 0..3
+    const uint32_t hi = (v >> 4) & 0x0F0F0F0Fu;  // nibbles 1, 3, 5, 7
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      // fp16 pair (nibble 2p, nibble 2p+1): low byte of each half from lo / hi byte p
+      const uint32_t sel = (uint32_t)(p) | (0x0Cu << 8) | ((uint32_t)(4 + p) << 16) | (0x0Cu << 24);
+      const uint32_t pr = __builtin_amdgcn_perm(hi, lo, sel) | 0x64006400u;
+      out[p] = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(h2, pr) - bias) * f.s);
+    }
+  } else {
+    const uint32_t a = w << 6, b = w << 2, c = w >> 2, d = w >> 6;
+    const uint32_t x[4] = {__builtin_amdgcn_perm(b, a, 0x05040100u), __builtin_amdgcn_perm(d, c, 0x05040100u),
+                           __builtin_amdgcn_perm(b, a, 0x07060302u), __builtin_amdgcn_perm(d, c, 0x07060302u)};
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      out[p] = __builtin_bit_cast(
+          uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, nib_pair(x[p])), f.mul, f.add));
   }
   return out;
+}
+
+// Eight fp16 values (column order) into pair order.
+__device__ __forceinline__ u32x4 to_pairs(const u32x4 v) {
+  return u32x4{__builtin_amdgcn_perm(v[2], v[0], 0x05040100u), __builtin_amdgcn_perm(v[2], v[0], 0x07060302u),
+               __builtin_amdgcn_perm(v[3], v[1], 0x05040100u), __builtin_amdgcn_perm(v[3], v[1], 0x07060302u)};
 }
 
 // Word s of lane row group G becomes word G of row group s (lane l % 16 kept).

@@ -19,9 +19,11 @@
 // lane, transposed across the four lane rows as in the skinny GEMM (q4d_gemm.hip).
 //
 // What bounds it: a few rows, the launch and one memory round trip (16 rows of 3072 x 1024
-// fp32: 3.3 us, 9.4 as 16 GEMVs); many, the unpacking and splitting VALU work per MFMA and
-// the activations' re-reads from L2 (211 rows of 1024 x 3072: 9.5 us, was 142; 1024 rows of
-// 3072 x 1024: 34 us, was 466).
+// fp32: 3.2 us, 9.4 as 16 GEMVs); many, the unpacking and splitting VALU work per MFMA and
+// the activations' re-reads from L2 (211 rows of 1024 x 3072: 9.1 us, was 142; 1024 rows of
+// 3072 x 1024: 32 us, was 466).
+#include <type_traits>
+
 #include "q4d_internal.h"
 #include "q4d_mfma_dev.h"
 
@@ -63,27 +65,36 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
     wo[j] = n * (a.K / 2) + 16 * G;
     so[j] = n * (a.K / 32);
   }
-  // activation loads of a unit: XL instructions, each CPR lanes of 16 bytes per row
-  constexpr int XB = XF32 ? 4 : 2, CPR = 8 * XB, RPI = 64 / CPR, XL = 16 * MT / RPI;
-  const int xr = lane / CPR, xc = lane % CPR;
+  // activation loads of a unit: 16 lanes per row, 8 columns each (fp32: two 16-byte loads)
+  constexpr int XB = XF32 ? 4 : 2, XR = 4 * MT, XL = XR * (XB / 2);
+  const int xr = lane >> 4, xc = lane & 15;
   const char* xb = static_cast<const char*>(a.x) + (size_t)m0 * a.K * XB;
-  uint32_t xo[XL];
+  uint32_t xo[XR];
 #pragma unroll
-  for (int i = 0; i < XL; ++i) xo[i] = (uint32_t)min(RPI * i + xr, a.M - 1 - m0) * a.K * XB + 16 * xc;
+  for (int i = 0; i < XR; ++i) xo[i] = (uint32_t)min(4 * i + xr, a.M - 1 - m0) * a.K * XB + 8 * XB * xc;
 
   struct Unit {
     u32x4 x[XL];
     u32x4 c[NT];
     uint32_t s[NT];
   } U[UPW > 0 ? UPW : 1];
+  auto load_scales = [&](Unit& L, int u) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) L.s[j] = *reinterpret_cast<const uint32_t*>(sb + 4 * u + so[j]);
+  };
   auto load = [&](Unit& L, int u) {
 #pragma unroll
-    for (int i = 0; i < XL; ++i) L.x[i] = *reinterpret_cast<const u32x4*>(xb + u * (kRwUnit * XB) + xo[i]);
+    for (int i = 0; i < XL; ++i)
+      L.x[i] = *reinterpret_cast<const u32x4*>(xb + u * (kRwUnit * XB) + xo[i / (XB / 2)] + 16 * (i % (XB / 2)));
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      L.c[j] = *reinterpret_cast<const u32x4*>(wb + u * (kRwUnit / 2) + wo[j]);
-      L.s[j] = *reinterpret_cast<const uint32_t*>(sb + 4 * u + so[j]);
-    }
+    for (int j = 0; j < NT; ++j) L.c[j] = *reinterpret_cast<const u32x4*>(wb + u * (kRwUnit / 2) + wo[j]);
+  };
+  // whether a unit's weights need the general fp16 conversion (a scale code past the fast one)
+  auto wide_codes = [&](const Unit& L) {
+    uint32_t most = 0;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) most = max(most, max(L.s[j] & 0xFFFFu, L.s[j] >> 16));
+    return most;
   };
   f32x4 tot[MT][NT];
 #pragma unroll
@@ -91,26 +102,26 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
 #pragma unroll
     for (int j = 0; j < NT; ++j) tot[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  auto step = [&](Unit& L, int u) {
-    // activations to LDS: row RPI i + xr, hi at 0, lo 16 MT rows further
+  auto step = [&](Unit& L, int u, auto wide) {
+    // activations to LDS in pair order: row 4 i + xr, hi at 0, lo 16 MT rows further
 #pragma unroll
-    for (int i = 0; i < XL; ++i) {
-      _Float16* d = xs + (RPI * i + xr) * kRwLd + xc * (16 / XB);
+    for (int i = 0; i < XR; ++i) {
+      u32x4* d = reinterpret_cast<u32x4*>(xs + (4 * i + xr) * kRwLd + 8 * xc);
       if constexpr (XF32) {
-        uint32_t hw[2], lw[2];
+        u32x4 hw, lw;
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          const uint32_t b0 = L.x[i][2 * p], b1 = L.x[i][2 * p + 1];
+        for (int p = 0; p < 4; ++p) {
+          const uint32_t b0 = L.x[2 * i][p], b1 = L.x[2 * i + 1][p];
           const float f0 = __builtin_bit_cast(float, b0), f1 = __builtin_bit_cast(float, b1);
           const h2 h = make_h2((_Float16)f0, (_Float16)f1);
           hw[p] = __builtin_bit_cast(uint32_t, h);
           if constexpr (XP == 2)
             lw[p] = __builtin_bit_cast(uint32_t, make_h2((_Float16)(f0 - (float)h.x), (_Float16)(f1 - (float)h.y)));
         }
-        *reinterpret_cast<u32x2*>(d) = u32x2{hw[0], hw[1]};
-        if constexpr (XP == 2) *reinterpret_cast<u32x2*>(d + 16 * MT * kRwLd) = u32x2{lw[0], lw[1]};
+        *d = hw;
+        if constexpr (XP == 2) d[16 * MT * kRwLd / 8] = lw;
       } else {
-        *reinterpret_cast<u32x4*>(d) = L.x[i];
+        *d = to_pairs(L.x[i]);
       }
     }
     uint32_t d4[NT][4], sc[NT];
@@ -120,18 +131,18 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) d4[j][e] = L.c[j][e];
     }
-    if (UPW == 0 && u + 1 < u1) load(L, u + 1);
+    if (UPW == 0 && u + 1 < u1) {
+      load_scales(L, u + 1);
+      load(L, u + 1);
+    }
 #pragma unroll
     for (int j = 0; j < NT; ++j) rows_transpose4(d4[j]);
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
-      h2 sh[NT];
+      W16Scale sh[NT];
       if constexpr (XP == 0) {
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          const _Float16 f = (_Float16)scale_q2_14(g ? sc[j] >> 16 : sc[j] & 0xFFFFu);
-          sh[j] = make_h2(f, f);
-        }
+        for (int j = 0; j < NT; ++j) sh[j] = w16_scale(g ? sc[j] >> 16 : sc[j] & 0xFFFFu);
       }
       f32x4 p[MT][NT];
 #pragma unroll
@@ -150,13 +161,13 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
           if constexpr (XP == 0) {
-            const h8 q = __builtin_bit_cast(h8, dequant8(d4[j][s], sh[j]));
+            const h8 q = __builtin_bit_cast(h8, dequant8_pairs<decltype(wide)::value>(d4[j][s], sh[j]));
 #pragma unroll
             for (int i = 0; i < MT; ++i)
               tot[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[i], q, tot[i][j], 0, 0, 0);
             continue;
           }
-          const h8 q = __builtin_bit_cast(h8, codes8(d4[j][s]));
+          const h8 q = __builtin_bit_cast(h8, codes8_pairs(d4[j][s]));
 #pragma unroll
           for (int i = 0; i < MT; ++i) {
             p[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[i], q, p[i][j], 0, 0, 0);
@@ -167,7 +178,7 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
       if constexpr (XP == 0) continue;
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
-        const float f = scale_q2_14(g ? sc[j] >> 16 : sc[j] & 0xFFFFu);
+        const float f = 8.0f * scale_q2_14(g ? sc[j] >> 16 : sc[j] & 0xFFFFu);  // the codes are q / 8
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -175,14 +186,35 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
       }
     }
   };
+  constexpr bool kWideOnly = XP == 0 && MT * NT >= 8 && UPW > 1;
+  const auto units = [&](auto wide) {
+#pragma unroll
+    for (int d = 0; d < UPW; ++d) step(U[d], u0 + d, wide);
+  };
   if constexpr (UPW > 0) {
+    // the scales first: the choice of conversion waits for them alone
+#pragma unroll
+    for (int d = 0; d < UPW; ++d) load_scales(U[d], u0 + d);
 #pragma unroll
     for (int d = 0; d < UPW; ++d) load(U[d], u0 + d);
+    uint32_t most = 0;
 #pragma unroll
-    for (int d = 0; d < UPW; ++d) step(U[d], u0 + d);
-  } else {
-    if (u0 < u1) load(U[0], u0);
-    for (int u = u0; u < u1; ++u) step(U[0], u);
+    for (int d = 0; d < UPW; ++d) most = max(most, wide_codes(U[d]));
+    // (the largest tile over several units: the general conversion always; two copies of that
+    // much code cost more than it saves: 768 x 1024 x 3072 17.4 us, 19.2 with both)
+    if (XP == 0 && (kWideOnly || scale_wide(most)))
+      units(std::true_type{});
+    else if constexpr (!kWideOnly)
+      units(std::false_type{});
+  } else if (u0 < u1) {
+    load_scales(U[0], u0);
+    load(U[0], u0);
+    for (int u = u0; u < u1; ++u) {
+      if (XP == 0 && scale_wide(wide_codes(U[0])))
+        step(U[0], u, std::true_type{});
+      else
+        step(U[0], u, std::false_type{});
+    }
   }
 
   // lane holds activation rows 16 i + 4G + r of weight row 16 j + l % 16

@@ -11,10 +11,15 @@ from llm_accelerator_amd.model import KVCache, Qwen3Config, build_model, random_
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module")
-def model(dev):
+@pytest.fixture(scope="module", params=["usual scales", "wide scales"])
+def model(dev, request):
     cfg = Qwen3Config(num_hidden_layers=2, vocab_size=4096)
-    return build_model(cfg, random_host_weights(cfg, seed=21), 1024, dev)
+    host = random_host_weights(cfg, seed=21)
+    if request.param == "wide scales":  # codes past the fast conversion's limit in some groups
+        for L in host["layers"]:
+            for name in ("q_proj", "o_proj", "up_proj", "down_proj"):
+                L[name][1][5::64, 3::7] = 4095 + L[name][1][5::64, 3::7]
+    return build_model(cfg, host, 1024, dev)
 
 
 @pytest.fixture(scope="module")

@@ -80,15 +80,18 @@ def test_linear_group_rows_equal_single_calls(dev):
         assert torch.equal(y, linear(w, x))
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 128, 1024), (33, 1024, 3072), (64, 384, 2048), (100, 3072, 1024), (500, 3072, 1024),
-                                   (401, 1024, 3072), (64, 128, 1152)])
-def test_gemm_few_outputs_vs_fp16_operands(dev, m, n, k):
-    """q4d_gemm where it takes the rows kernel: the product of the same fp16 operands (weights
-    rounded once), every tile size and the general K loop (1152 columns)."""
+@pytest.mark.parametrize("m,n,k,top", [(1, 128, 1024, 1500), (33, 1024, 3072, 1500), (64, 384, 2048, 9000),
+                                       (100, 3072, 1024, 4095), (500, 3072, 1024, 1500), (401, 1024, 3072, 1500),
+                                       (64, 128, 1152, 65535), (700, 4096, 1024, 9000), (2000, 1024, 2048, 9000)])
+def test_gemm_vs_fp16_operands(dev, m, n, k, top):
+    """q4d_gemm against the product of the same fp16 operands (weights rounded once): the rows
+    kernel's tile sizes and general K loop (1152 columns), the tiled and the pipelined kernel,
+    with scale codes on both sides of the fast conversion's limit (4094)."""
     from llm_accelerator_amd.model import current_stream
     rng = np.random.default_rng(m + n + k)
     packed = rng.integers(0, 256, size=(n, k // 2), dtype=np.uint8)
-    scale = rng.integers(1, 1500, size=(n, k // 64)).astype(np.uint16)
+    scale = rng.integers(1, top + 1, size=(n, k // 64)).astype(np.uint16)
+    scale[0, :2] = min(top, 4094), top
     w = q4(packed, scale, dev)
     x = torch.from_numpy(rng.normal(size=(m, k)).astype(np.float16)).to(dev)
     resid = torch.from_numpy(rng.normal(size=(m, n)).astype(np.float32)).to(dev)
@@ -99,5 +102,6 @@ def test_gemm_few_outputs_vs_fp16_operands(dev, m, n, k):
     q = o.unpack_signed_int4(packed, k).astype(np.float16)
     w16 = (q * np.repeat((scale / 16384.0).astype(np.float16), 64, axis=1)).astype(np.float64)
     x64 = x.double().cpu().numpy()
+    assert np.isfinite(w16).all()
     bound = 2.0 ** -16 * (np.abs(x64) @ np.abs(w16).T) + 2.0 ** -22
     assert np.all(np.abs(y.double().cpu().numpy() - resid.double().cpu().numpy() - x64 @ w16.T) <= bound)
