@@ -662,13 +662,24 @@ int q4d_gemm_splitk(const q4d_matrix_t* w, const uint16_t* x, int32_t M, void* y
   return launch_gemm(a, resid ? EP_RESID : (y_dtype == Q4D_F16 ? EP_F16 : EP_F32), false, as_stream(stream));
 }
 
-// Final RMSNorm (to fp16) + LM head GEMM with per-row argmax partials over
-// 128-column blocks + one wave per row reducing them.
+// Final RMSNorm (to fp16) + LM head GEMM with per-row argmax partials per block + one wave
+// per row reducing them: up to 64 rows in the resident kernel of q4d_lm_batch.hip, more on
+// the tiled GEMM (partials over 128-column blocks).
 static int run_lm_head_batch(const q4d_model_t* model, const float* hidden, int batch, int32_t* next_tokens,
                              float* scores, float* logits, void* ws, const WsLayout& W, hipStream_t st) {
   const int H = model->hidden_size;
   uint16_t* xh = ws_ptr<uint16_t>(ws, W.xh);
-  int rc = launch_rms_norm(hidden, model->final_norm, model->rms_norm_eps, batch, H, xh, Q4D_F16, st);
+  float* part_score = ws_ptr<float>(ws, W.row_score);
+  int* part_idx = ws_ptr<int>(ws, W.row_idx);
+  int rc;
+  const LmBatchArgs lb = {model->embed_tokens.w, model->embed_tokens.s, hidden, model->final_norm, model->rms_norm_eps,
+                          logits, part_score, part_idx, batch, model->vocab_size};
+  if (lm_batch_applies(lb, H)) {
+    int nparts = 0;
+    if ((rc = launch_lm_batch(lb, &nparts, st))) return rc;
+    return launch_argmax_rows(part_score, part_idx, nparts, batch, next_tokens, scores, st);
+  }
+  rc = launch_rms_norm(hidden, model->final_norm, model->rms_norm_eps, batch, H, xh, Q4D_F16, st);
   if (rc) return rc;
   GemmArgs g;
   memset(&g, 0, sizeof(g));
@@ -681,8 +692,8 @@ static int run_lm_head_batch(const q4d_model_t* model, const float* hidden, int 
   g.M = batch;
   g.x = xh;
   g.logits = logits;
-  g.part_score = ws_ptr<float>(ws, W.row_score);
-  g.part_idx = ws_ptr<int>(ws, W.row_idx);
+  g.part_score = part_score;
+  g.part_idx = part_idx;
   if ((rc = launch_gemm(g, EP_ARGMAX, false, st))) return rc;
   return launch_argmax_rows(g.part_score, g.part_idx, model->vocab_size / 128, batch, next_tokens, scores, st);
 }

@@ -391,6 +391,24 @@ int launch_splitk_resid_norm(const GemmArgs& a, int ksplit, const float* gamma, 
 int launch_argmax_rows(const float* part_score, const int* part_idx, int nparts, int M, int32_t* out_token,
                        float* out_score, hipStream_t st);
 
+// ---- batched LM head (q4d_lm_batch.hip) ---------------------------------------
+// Final RMSNorm of M <= 64 fp32 rows, the tied table on MFMA (fp16 operands) and per-row
+// argmax partials [M][*nparts], *nparts <= N / 128, for launch_argmax_rows; logits [M, N]
+// optional.
+struct LmBatchArgs {
+  const uint8_t* w;
+  const uint16_t* s;
+  const float* hidden;  // [M, 1024]
+  const float* gamma;
+  float eps;
+  float* logits;
+  float* part_score;
+  int* part_idx;
+  int M, N;
+};
+bool lm_batch_applies(const LmBatchArgs& a, int K);
+int launch_lm_batch(const LmBatchArgs& a, int* nparts, hipStream_t st);
+
 // ---- integer Q4 GEMV of the fixed-point path (q4d_int.hip) ------------------
 int launch_gemv_q26(const q4d_matrix_t* w, const int32_t* x, int64_t* y_q26, int32_t* y_q12, int32_t* saturated,
                     hipStream_t st);
