@@ -410,36 +410,94 @@ __global__ __launch_bounds__(256) void attn_kernel(const AttnArgs a) {
   if (t == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // next launch
 }
 
+// Inclusive sum over the lanes of a wave (DPP row shifts, then the row totals).
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr 1, 2, 4, 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast 15 into rows 1, 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast 31 into rows 2, 3
+  return x;
+}
+
+constexpr int kSpanSplits = 16;  // splits of one sequence at most
+constexpr int kSpanMerge = 8;    // splits merged in one batch of loads
+
+// Which part of which sequence block `idx` of a kv head takes.
+struct SpanWork {
+  int b, s, nsplit, pos;  // b < 0: none
+};
+
+// Every sequence is cut into round(its sub-chunks / S) parts, at least one, with
+// S = ceil(all sub-chunks / slots): the parts number at most slots + batch, which is the
+// launcher's grid.  Rounded up, the sequences a little longer than S became two short parts
+// and a merge (64 x 285-600 positions: 23.9 us, 21.4 as one part each).  More than eight
+// parts of one sequence cost a second batch of merge loads, so they have four sub-chunks or
+// more each.  Batches of `slots` sequences and more are one part per sequence, without the
+// cut's ~0.4 us (64 sequences: equal lengths 43.2 against 43.6 us, 47-2000 positions 48.1
+// against 49.4).  A position out of range counts as one part of no sub-chunks, whose
+// block reports it.  Every wave of every block computes the same split from the positions
+// (lane l: sequence g + l).
+__device__ __forceinline__ SpanWork span_work(const AttnArgs& a, int idx, int slots, int lane) {
+  if (a.batch >= slots) return {idx, 0, 1, a.positions[idx]};
+  const auto load = [&](int b) { return b < a.batch ? a.positions[b] : -1; };
+  const auto subs = [&](int p) { return p >= 0 && p < a.max_ctx ? p / kAttnChunk + 1 : 0; };
+  int p = load(lane);
+  int total = __builtin_amdgcn_readlane(wave_scan(subs(p)), 63);
+  for (int g = kWave; g < a.batch; g += kWave) total += __builtin_amdgcn_readlane(wave_scan(subs(load(g + lane))), 63);
+  const int S = max(1, (total + slots - 1) / slots);
+  for (int g = 0;;) {
+    const int n0 = subs(p), most = max(kSpanMerge, min(kSpanSplits, n0 / 4));
+    const int ns = g + lane < a.batch ? min(most, max(1, (n0 + S / 2) / S)) : 0;
+    const int incl = wave_scan(ns);
+    const int all = __builtin_amdgcn_readlane(incl, 63);
+    if (idx < all) {
+      const int l = __builtin_ctzll(__ballot(incl > idx));
+      const int n = __builtin_amdgcn_readlane(ns, l);
+      return {g + l, idx - __builtin_amdgcn_readlane(incl, l) + n, n, __builtin_amdgcn_readlane(p, l)};
+    }
+    idx -= all;
+    g += kWave;
+    if (g >= a.batch) return {-1, 0, 0, 0};
+    p = load(g + lane);
+  }
+}
+
 // Long-context variant of attn_kernel<64> with merge = 1 (batched decode,
-// q4d_cached_attention): a block covers one of nsplit nearly equal parts of the
-// T = pos + 1 positions (nsplit = ceil(T / span), parts of whole 64-position
-// sub-chunks) as consecutive sub-chunks, with the next sub-chunk's K/V loads
-// in flight while the current one is used.  Each wave keeps its own online
-// softmax (running maximum M and sum L per head; its output accumulators are
-// rescaled by 2^(M_old - M_new) when M grows) over its 16 positions of every
-// sub-chunk, so the sub-chunk loop has no barrier; the four waves' states are
-// merged once after the span.  K/V are read with non-temporal loads (read once
-// per step).  The launcher sizes `span` for about two blocks per CU over the
-// batch's (sequence, kv head) pairs: a few long contiguous K/V streams per CU
-// read HBM faster than many short ones (64 x 4097 positions, 28 layers: eight
-// 576-position spans per head, 5 resident blocks per CU and 32-position
-// sub-chunks took 6.35 ms per step; equal parts 6.27; one block per head with
-// 64-position sub-chunks 5.48).  Same prologue and partial format as
-// attn_kernel<64>; thread t owns dims 8 (t % 16) .. +7 of positions t / 16 + 16 i.
-__global__ __launch_bounds__(256) void attn_span_kernel(const AttnArgs a, int span) {
+// q4d_cached_attention): a block covers one of a sequence's nsplit nearly equal
+// parts of its T = pos + 1 positions (parts of whole 64-position sub-chunks) as
+// consecutive sub-chunks, with the next sub-chunk's K/V loads in flight while the
+// current one is used.  Each wave keeps its own online softmax (running maximum M
+// and sum L per head; its output accumulators are rescaled by 2^(M_old - M_new)
+// when M grows) over its 16 positions of every sub-chunk, so the sub-chunk loop has
+// no barrier; the four waves' states are merged once after the span.  K/V are read
+// with non-temporal loads (read once per step).  The parts are cut from the
+// sequences' own positions (span_work) to about two blocks per CU of nearly equal
+// length: a few long contiguous K/V streams per CU read HBM faster than many short
+// ones (64 x 4097 positions, 28 layers: eight 576-position spans per head, 5
+// resident blocks per CU and 32-position sub-chunks took 6.35 ms per step; equal
+// parts 6.27; one block per head with 64-position sub-chunks 5.48).
+// Cut from the capacity instead, as before, one long part held up ragged batches and short
+// contexts of a large cache ran on few blocks (us a call, before / now): 24 x 649-1500
+// positions 24.8 / 21.8, 8 x 2000 of 8192 31.0 / 17.8, 40 x 660-3000 of 4096 63.6 / 55.8, one
+// sequence of 8000 18.4 / 13.4; uniform batches that fill the cache within 2 %.
+// Same prologue and partial format as attn_kernel<64>; thread t owns dims
+// 8 (t % 16) .. +7 of positions t / 16 + 16 i.
+__global__ __launch_bounds__(256) void attn_span_kernel(const AttnArgs a, int slots) {
   attn_preload(a);
-  constexpr int D = 128, CH = 64, NPT = CH / 16;
-  const int s = blockIdx.x, j = blockIdx.y, b = blockIdx.z;
+  constexpr int D = 128, CH = kAttnChunk, NPT = CH / 16;
   const int t = threadIdx.x, lane = t & 63;
   const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int pos = a.positions[b];
+  const int idx = blockIdx.x / a.kvh, j = blockIdx.x - idx * a.kvh;
+  const SpanWork wk = span_work(a, idx, slots, lane);
+  const int b = wk.b, s = wk.s, nsplit = wk.nsplit, pos = wk.pos;
+  if (b < 0) return;
   if (pos < 0 || pos >= a.max_ctx) {
-    if (s == 0 && j == 0 && t == 0) atomicOr(a.status, Q4D_STATUS_BAD_POSITION);
+    if (j == 0 && t == 0) atomicOr(a.status, Q4D_STATUS_BAD_POSITION);
     return;
   }
   const int T = pos + 1;
-  const int nsplit = (T + span - 1) / span;
-  if (s >= nsplit) return;
   const int nsub_all = (T + CH - 1) / CH;
   const int start = (s * nsub_all / nsplit) * CH;
   const int end = min(T, ((s + 1) * nsub_all / nsplit) * CH);
@@ -677,7 +735,7 @@ __global__ __launch_bounds__(256) void attn_span_kernel(const AttnArgs a, int sp
   if (t == 0) s_last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nsplit - 1;
   __syncthreads();
   if (!s_last) return;
-  constexpr int kMergeBatch = 8;
+  constexpr int kMergeBatch = kSpanMerge;
   float Mx = -INFINITY, Lx = 0.f, o = 0.f;
   for (int i0 = 0; i0 < nsplit; i0 += kMergeBatch) {
     float mi[kMergeBatch], li[kMergeBatch], ai[kMergeBatch];
@@ -710,19 +768,17 @@ __global__ __launch_bounds__(256) void attn_span_kernel(const AttnArgs a, int sp
 int launch_attention(const AttnArgs& a, hipStream_t stream) {
   if (!a.part_ml || !a.part_acc || (a.merge && !a.counters)) return Q4D_ERR_NULL;
   if (a.merge) {
-    // contexts past kSpanSplits x 64 positions: spans of several 64-position
-    // sub-chunks, at most kSpanSplits per head, as many as make about two blocks
-    // per CU over the (sequence, kv head) pairs
-    constexpr int kSpanSplits = 8;
+    // contexts past 512 positions: the sequences' positions are on the device, so the
+    // grid is the bound of span_work's parts and blocks past the last part end at once
     const int nch = (a.max_ctx + kAttnChunk - 1) / kAttnChunk;
-    if (nch <= kSpanSplits) {
+    if (nch <= kSpanMerge) {
       hipLaunchKernelGGL(attn_kernel<kAttnChunk>, dim3(a.nsplit_max, a.kvh, a.batch), dim3(256), 0, stream, a);
     } else {
-      const int pairs = a.batch * a.kvh;
-      const int ns = max(1, min(kSpanSplits, (2 * device_cus() + pairs - 1) / pairs));
-      const int span = kAttnChunk * ((nch + ns - 1) / ns);
-      const int nsplit = (a.max_ctx + span - 1) / span;
-      hipLaunchKernelGGL(attn_span_kernel, dim3(nsplit, a.kvh, a.batch), dim3(256), 0, stream, a, span);
+      const int slots = max(1, 2 * device_cus() / a.kvh);
+      const long long parts = a.batch >= slots
+                                  ? a.batch
+                                  : min((long long)a.batch * min(kSpanSplits, nch), (long long)a.batch + slots);
+      hipLaunchKernelGGL(attn_span_kernel, dim3((unsigned)(parts * a.kvh)), dim3(256), 0, stream, a, slots);
     }
   } else if (a.chunk == kAttnChunk) {
     const int ns = (a.max_ctx + kAttnChunk - 1) / kAttnChunk;
