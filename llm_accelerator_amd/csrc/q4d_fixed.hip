@@ -348,8 +348,13 @@ __global__ __launch_bounds__(256) void fx_gemv_kernel(const FxGemv a) {
 //     floor((e << 16) / sum)) into LDS, then sum_p prob_p * v_p for the block's 32 dims,
 //     exact in int64, and sat24(sum >> 16).  Every block of a head recomputes the same
 //     softmax (T scores and at most 16 maxima), which costs less than handing it over.
+//     What bounds it is the chain of memory round trips on 64 blocks: the first 1024
+//     positions' V rows are all in flight before the softmax (kFxAhead rounds; one round of
+//     256 at a time: 8.45 us a layer at position 700, now 7.5; a token 882 -> 862 us).
+//     Blocks of 1024 threads with one V round were slower (921 us a token).
 // The kernel boundary orders the workspace traffic; no counters or device-scope atomics.
 constexpr int kFxMaxChunks = 16;
+constexpr int kFxAhead = 4;  // rounds of 256 V rows that fx_attn_value has in flight
 
 struct FxAttn {
   const int32_t* qkv;       // FULL: q|k|v projections of this token
@@ -526,23 +531,23 @@ __global__ __launch_bounds__(256) void fx_attn_value_kernel(const FxAttn a) {
   if (!fx_attn_pos<FULL>(a, pos)) return;
   const int T = pos + 1, nct = (T + a.ch - 1) / a.ch;
 
-  // loads in the order they are consumed: chunk maxima, scores, LUT, then the first round
-  // of V rows (thread = 4 dims x position residue mod 32)
+  // loads in the order they are consumed: chunk maxima, scores, LUT, then the first
+  // kFxAhead rounds of V rows (thread = 4 dims x position residue mod 32)
   long long cmv[kFxMaxChunks];
 #pragma unroll
   for (int i = 0; i < kFxMaxChunks; ++i) cmv[i] = a.cmax[h * kFxMaxChunks + (i < nct ? i : nct - 1)];
   constexpr int NP = kFxMaxCtx / 256;  // score positions per thread
   long long sv[NP];
 #pragma unroll
-  for (int k = 0; k < NP; ++k) {  // clamped: slots past the context re-read the last score
+  for (int k = 0; k < NP; ++k) {  // clamped to the last score; slots past the context are skipped whole
     const int p = t + 256 * k;
-    sv[k] = a.sc[(size_t)h * a.max_ctx + (p < T ? p : T - 1)];
+    sv[k] = 256 * k < T ? a.sc[(size_t)h * a.max_ctx + (p < T ? p : T - 1)] : 0;
   }
   for (int i = t; i < kFxExpLut; i += 256) lut[i] = a.exp_lut[i];
   const int dq = t & 7, j = t >> 3;
   const int32_t* vbase = a.vc + (size_t)g * a.max_ctx * 128 + 32 * db + 4 * dq;
-  i32x4 v4[8];
-  auto load_v = [&](int p0) {
+  i32x4 v4[kFxAhead][8];
+  auto load_v = [&](i32x4(&v4)[8], int p0) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int p = p0 + 32 * u;
@@ -550,7 +555,9 @@ __global__ __launch_bounds__(256) void fx_attn_value_kernel(const FxAttn a) {
     }
   };
   __builtin_amdgcn_sched_barrier(0);
-  load_v(j);
+#pragma unroll
+  for (int r = 0; r < kFxAhead; ++r)
+    if (256 * r < T) load_v(v4[r], j + 256 * r);
   __builtin_amdgcn_sched_barrier(0);
 
   // softmax (46_...:96-121)
@@ -594,7 +601,7 @@ __global__ __launch_bounds__(256) void fx_attn_value_kernel(const FxAttn a) {
 
   // value sums (46_...:124-137) for dims 32 db + 4 dq .. + 3
   long long acc0 = 0, acc1 = 0, acc2 = 0, acc3 = 0;
-  auto value_round = [&](int p0) {
+  auto value_round = [&](const i32x4(&v4)[8], int p0) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int p = p0 + 32 * u;
@@ -605,10 +612,12 @@ __global__ __launch_bounds__(256) void fx_attn_value_kernel(const FxAttn a) {
       acc3 += pr * v4[u].w;
     }
   };
-  value_round(j);
-  for (int p0 = j + 256; p0 < T; p0 += 256) {
-    load_v(p0);
-    value_round(p0);
+#pragma unroll
+  for (int r = 0; r < kFxAhead; ++r)
+    if (256 * r < T) value_round(v4[r], j + 256 * r);
+  for (int p0 = 256 * kFxAhead; p0 < T; p0 += 256) {
+    load_v(v4[0], j + p0);
+    value_round(v4[0], j + p0);
   }
   // the 8 residues of a wave sit in lanes dq + 8 r: reduce over r, then over the 4 waves
 #pragma unroll
