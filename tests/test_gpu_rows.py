@@ -51,6 +51,22 @@ def test_linear_rows_vs_oracle(dev, m, n, k, xdtype, ydtype, precision):
     assert np.all((np.abs(y - ref) <= ACC * size + xerr + out)[finite])
 
 
+@pytest.mark.parametrize("m,n,k", [(20, 256, 3072), (60, 3072, 3072), (211, 1024, 3072), (600, 3072, 2048), (50, 1024, 2048)])
+def test_linear_rows_integer_exact(dev, m, n, k):
+    """Several 128-column units per wave through the same LDS rows (two and three per wave, and the
+    general loop of the largest tile), integers small enough that every sum is exact: equal bits, so a
+    row read before the wave's other lanes have stored it, or after the next unit's, shows."""
+    rng = np.random.default_rng(m + n + k)
+    packed = o.pack_signed_int4(rng.integers(-8, 8, size=(n, k)))
+    scale = rng.integers(1, 32, size=(n, k // 64)).astype(np.uint16)
+    x = rng.integers(-4, 5, size=(m, k)).astype(np.float32)
+    W = o.dequantize_q4(packed, scale, dtype=np.float64)
+    assert (np.abs(x).astype(np.float64) @ np.abs(W).T).max() < 1024  # multiples of 2^-14: exact in fp32
+    print(f"[linear rows exact] {m} x {n} x {k}", flush=True)
+    y = linear(q4(packed, scale, dev), torch.from_numpy(x).to(dev)).cpu().numpy()
+    np.testing.assert_array_equal(y, (x.astype(np.float64) @ W.T).astype(np.float32))
+
+
 def test_linear_rows_one_bad_row_stays_alone(dev):
     """A row holding an infinity or a NaN does not reach the other rows of its tile."""
     rng = np.random.default_rng(3)
