@@ -848,13 +848,8 @@ int launch_gemv_group(int rows, int cols, int batch, const uint8_t* const* w, co
     if (!w[i] || !s[i] || !x[i] || !y[i]) return Q4D_ERR_NULL;
     if (!aligned(w[i], 16) || !aligned(s[i], 4) || !aligned(x[i], 16)) return Q4D_ERR_BAD_ADDR;
   }
-  if (batch >= kRowsMin) {  // as q4d_linear: each matrix fills the device by itself
-    for (int i = 0; i < count; ++i) {
-      const int rc = launch_rows(RowsArgs{w[i], s[i], x[i], y[i], nullptr, batch, rows, cols}, xm == X_F32, xp, ep, st);
-      if (rc) return rc;
-    }
-    return Q4D_OK;
-  }
+  if (batch >= kRowsMin)  // as q4d_linear
+    return launch_rows_group(batch, rows, cols, w, s, x, y, count, xm == X_F32, xp, ep, st);
   GemvGroupArgs G;
   memset(&G, 0, sizeof(G));
   G.a.rows = rows;

@@ -212,6 +212,17 @@ struct RowsArgs {
   int M, N, K;
 };
 int launch_rows(const RowsArgs& a, bool xf32, int xp, int ep, hipStream_t st);
+// The same over `count` matrices of one shape, each with its own x and y, up to 64 a launch:
+// every y[i] equals its own launch_rows bit for bit.  xp 1 or 2, ep EP_F16 / EP_F32.
+int launch_rows_group(int M, int N, int K, const uint8_t* const* w, const uint16_t* const* s, const void* const* x,
+                      void* const* y, int count, bool xf32, int xp, int ep, hipStream_t st);
+// The block's tile of 16 mt activation rows x 16 nt weight rows for `count` matrices in a
+// launch; k12: K = 3072 over 12 waves instead of 8.
+struct RowsTile {
+  int mt, nt;
+  bool k12;
+};
+RowsTile rows_tile(int M, int N, int K, int count);
 // Activation rows from which q4d_linear takes this kernel instead of one GEMV per row
 // (3072 x 1024 / 1024 x 3072, fp32: 3 rows 3.7 / 4.5 us as GEMVs; 4 rows 4.0 / 5.0 against
 // 3.2 / 5.1 here, 8 rows 5.8 / 8.0 against 3.2 / 5.1).

@@ -35,13 +35,30 @@ constexpr int kRwUnit = 128;           // K columns per wave and step
 constexpr int kRwLd = kRwUnit + 16;    // LDS row stride in fp16: 288 B, conflict-free MFMA operand reads
 constexpr int kRwRed = 17;             // LDS row stride (floats) of the partial tiles
 
+// Up to kRowsGroupMax matrices of one shape in a launch (matrix blockIdx.z); a's pointers unused.
+constexpr int kRowsGroupMax = 64;
+struct RowsGroupArgs {
+  RowsArgs a;
+  const uint8_t* w[kRowsGroupMax];
+  const uint16_t* s[kRowsGroupMax];
+  const void* x[kRowsGroupMax];
+  void* y[kRowsGroupMax];
+};
+
+__device__ __forceinline__ RowsArgs rows_of(const RowsArgs& a) { return a; }
+__device__ __forceinline__ RowsArgs rows_of(const RowsGroupArgs& g) {
+  const int z = blockIdx.z;
+  return RowsArgs{g.w[z], g.s[z], g.x[z], g.y[z], nullptr, g.a.M, g.a.N, g.a.K};
+}
+
 // XF32: fp32 activations (else fp16).  XP: 2 = hi + lo halves, 1 = one fp16 value, 0 = one fp16
 // value and the weights rounded to fp16 as q4d_gemm states it (one rounding of code x scale,
 // so no scale is applied to the sums).  The block's
 // tile is 16 MT activation rows x 16 NT weight rows.  UPW > 0: every wave has UPW units and
 // issues all their loads at entry; 0: any number, the next unit's loads in flight.
-template <bool XF32, int XP, int EP, int MT, int NT, int NW, int UPW>
-__global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
+template <bool XF32, int XP, int EP, int MT, int NT, int NW, int UPW, class Args>
+__global__ __launch_bounds__(NW * 64) void rows_kernel(const Args args) {
+  const RowsArgs a = rows_of(args);
   static_assert(XF32 ? XP != 0 : XP != 2, "fp16 activations are one value");
   constexpr int kH = XP == 2 ? 2 : 1;
   constexpr int kX = NW * kH * 16 * MT * kRwLd * 2, kR = NW * MT * NT * 16 * kRwRed * 4;
@@ -251,51 +268,83 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const RowsArgs a) {
   }
 }
 
-template <bool XF32, int XP, int EP, int MT, int NT>
-int launch_tile(const RowsArgs& a, hipStream_t st) {
-  const dim3 grid((a.N + 16 * NT - 1) / (16 * NT), (a.M + 16 * MT - 1) / (16 * MT));
-  const auto go = [&](auto kernel, int nw) { hipLaunchKernelGGL(kernel, grid, dim3(64 * nw), 0, st, a); };
+template <bool XF32, int XP, int EP, int MT, int NT, class Args>
+int launch_tile(const Args& args, const RowsArgs& a, int count, bool k12, hipStream_t st) {
+  const dim3 grid((a.N + 16 * NT - 1) / (16 * NT), (a.M + 16 * MT - 1) / (16 * MT), count);
+  const auto go = [&](auto kernel, int nw) { hipLaunchKernelGGL(kernel, grid, dim3(64 * nw), 0, st, args); };
   // Every unit of a wave in flight where K is one of the projections' widths and the
-  // registers hold them (211 x 1024 x 3072, hi + lo: 9.5 us, 11.5 with the next unit only);
-  // K = 3072 on one-tile blocks: 12 waves of two units (4 rows: 5.1 us, 5.5 with 8 of three).
-  constexpr bool kSmall = MT == 1 && NT == 1, kDeep = XP < 2 || MT * NT <= 4;
+  // registers hold them (211 x 1024 x 3072, hi + lo: 9.5 us, 11.5 with the next unit only).
+  constexpr bool kDeep = XP < 2 || MT * NT <= 4, kGroup = std::is_same_v<Args, RowsGroupArgs>;
+  constexpr bool k12Tile = MT == 1 && (NT == 1 || kGroup);  // the tiles that rows_tile gives 12 waves
   const int nu = a.K / kRwUnit;
+  if constexpr (k12Tile)
+    if (nu == 24 && k12) {
+      go(rows_kernel<XF32, XP, EP, MT, NT, 12, 2, Args>, 12);
+      return check_launch();
+    }
   if (nu == 8)
-    go(rows_kernel<XF32, XP, EP, MT, NT, 8, 1>, 8);
+    go(rows_kernel<XF32, XP, EP, MT, NT, 8, 1, Args>, 8);
   else if (nu == 16 && kDeep)
-    go(rows_kernel<XF32, XP, EP, MT, NT, 8, kDeep ? 2 : 0>, 8);
-  else if (nu == 24 && kSmall)
-    go(rows_kernel<XF32, XP, EP, MT, NT, kSmall ? 12 : 8, kSmall ? 2 : 0>, kSmall ? 12 : 8);
-  else if (nu == 24 && kDeep)
-    go(rows_kernel<XF32, XP, EP, MT, NT, 8, kDeep && !kSmall ? 3 : 0>, 8);
+    go(rows_kernel<XF32, XP, EP, MT, NT, 8, kDeep ? 2 : 0, Args>, 8);
+  else if (nu == 24 && kDeep && NT > 1)
+    go(rows_kernel<XF32, XP, EP, MT, NT, 8, (kDeep && NT > 1) ? 3 : 0, Args>, 8);
   else
-    go(rows_kernel<XF32, XP, EP, MT, NT, 8, 0>, 8);
+    go(rows_kernel<XF32, XP, EP, MT, NT, 8, 0, Args>, 8);
   return check_launch();
 }
 
 template <bool XF32, int XP, int EP>
 int launch_nt(const RowsArgs& a, hipStream_t st) {
-  // The largest tile (each split activation serves NT weight tiles, each unpacked weight MT
-  // row tiles) that still gives most CUs a block: 512 rows of 3072 x 1024, fp16: 24.4 us with
-  // MT = 1, 16.3 with 2; 64 rows of 2048 x 1024: 3.6 us on 256 blocks, 4.8 on 128.
-  const int mt = (a.M + 15) / 16, nt = (a.N + 15) / 16;
-  const auto blocks = [&](int m, int n) { return (long)((mt + m - 1) / m) * ((nt + n - 1) / n); };
-  constexpr long kMinBlocks = 192;
-  if (blocks(2, 4) >= kMinBlocks) return launch_tile<XF32, XP, EP, 2, 4>(a, st);
-  if (blocks(1, 4) >= kMinBlocks) return launch_tile<XF32, XP, EP, 1, 4>(a, st);
-  if (blocks(1, 2) >= kMinBlocks) return launch_tile<XF32, XP, EP, 1, 2>(a, st);
-  return launch_tile<XF32, XP, EP, 1, 1>(a, st);
+  const RowsTile t = rows_tile(a.M, a.N, a.K, 1);
+  if (t.mt == 2) return launch_tile<XF32, XP, EP, 2, 4>(a, a, 1, t.k12, st);
+  if (t.nt == 4) return launch_tile<XF32, XP, EP, 1, 4>(a, a, 1, t.k12, st);
+  if (t.nt == 2) return launch_tile<XF32, XP, EP, 1, 2>(a, a, 1, t.k12, st);
+  return launch_tile<XF32, XP, EP, 1, 1>(a, a, 1, t.k12, st);
+}
+
+template <bool XF32, int XP, int EP>
+int launch_group_nt(const RowsGroupArgs& g, int count, hipStream_t st) {
+  const RowsTile t = rows_tile(g.a.M, g.a.N, g.a.K, count);
+  if (t.mt == 2) return launch_tile<XF32, XP, EP, 2, 4>(g, g.a, count, t.k12, st);
+  if (t.nt == 4) return launch_tile<XF32, XP, EP, 1, 4>(g, g.a, count, t.k12, st);
+  return launch_tile<XF32, XP, EP, 1, 1>(g, g.a, count, t.k12, st);
 }
 
 }  // namespace
 
-int launch_rows(const RowsArgs& a, bool xf32, int xp, int ep, hipStream_t st) {
+// The largest tile (each split activation serves NT weight tiles, each unpacked weight MT row
+// tiles) that still gives most CUs a block: 512 rows of 3072 x 1024, fp16: 24.4 us with
+// MT = 1, 16.3 with 2; 64 rows of 2048 x 1024: 3.6 us on 256 blocks, 4.8 on 128.
+// One matrix of K = 3072 on one-tile blocks: 12 waves of two units (4 rows: 5.1 us, 5.5 with 8
+// of three), which groups the sums differently from 8 waves.  The matrices of a group count
+// together, but each keeps its own launch's waves, so its bits are its own launch's (12 waves
+// and two row tiles do not fit the LDS).
+RowsTile rows_tile(int M, int N, int K, int count) {
+  const int mt = (M + 15) / 16, nt = (N + 15) / 16;
+  const auto blocks = [&](int m, int n) { return (long)((mt + m - 1) / m) * ((nt + n - 1) / n); };
+  constexpr long kMinBlocks = 192;
+  RowsTile t = {1, 1, false};
+  if (blocks(2, 4) >= kMinBlocks) t = {2, 4, false};
+  else if (blocks(1, 4) >= kMinBlocks) t = {1, 4, false};
+  else if (blocks(1, 2) >= kMinBlocks) t = {1, 2, false};
+  else t.k12 = K == 24 * kRwUnit;
+  if (count > 1 && t.nt < 4 && blocks(1, 4) * count >= kMinBlocks) t.nt = 4;
+  if (count > 1 && !t.k12 && mt > 1 && blocks(2, 4) * count >= kMinBlocks) t = {2, 4, false};
+  return t;
+}
+
+static int check_rows(const RowsArgs& a, bool xf32, int xp, int ep) {
   if (!a.w || !a.s || !a.x || !a.y || (ep == EP_RESID && !a.resid)) return Q4D_ERR_NULL;
   if (a.M <= 0 || a.M > 16 * 65535 || a.N <= 0 || a.K <= 0 || a.K % kRwUnit) return Q4D_ERR_SHAPE;
   if (!aligned(a.w, 16) || !aligned(a.s, 4) || !aligned(a.x, 16)) return Q4D_ERR_BAD_ADDR;
   if (ep != EP_F16 && ep != EP_F32 && ep != EP_RESID) return Q4D_ERR_SHAPE;
   if (xf32 ? xp < 1 || xp > 2 : xp < 0 || xp > 1) return Q4D_ERR_DTYPE;
   if (ep == EP_RESID && (xf32 || xp)) return Q4D_ERR_DTYPE;
+  return Q4D_OK;
+}
+
+int launch_rows(const RowsArgs& a, bool xf32, int xp, int ep, hipStream_t st) {
+  if (const int rc = check_rows(a, xf32, xp, ep)) return rc;
   if (xf32 && xp == 2) return ep == EP_F16 ? launch_nt<true, 2, EP_F16>(a, st) : launch_nt<true, 2, EP_F32>(a, st);
   if (xf32) return ep == EP_F16 ? launch_nt<true, 1, EP_F16>(a, st) : launch_nt<true, 1, EP_F32>(a, st);
   if (xp == 1) return ep == EP_F16 ? launch_nt<false, 1, EP_F16>(a, st) : launch_nt<false, 1, EP_F32>(a, st);
@@ -304,6 +353,44 @@ int launch_rows(const RowsArgs& a, bool xf32, int xp, int ep, hipStream_t st) {
     case EP_F32: return launch_nt<false, 0, EP_F32>(a, st);
     default: return launch_nt<false, 0, EP_RESID>(a, st);
   }
+}
+
+// 64 fp32 matrices, us a call at 4 / 16 / 64 rows (a launch per matrix: 180-206 at K = 1024,
+// 317-380 at 3072, bound by the host; the grouped GEMV, which reads and unpacks a matrix again
+// for each row): 128 x 1024 5.0 / 6.5 / 11.1 (GEMV 5.5 / 13.8 / 47), 1024 x 1024 13.7 / 16.4 /
+// 50.7 (25 / 89 / 318), 3072 x 1024 32 / 35 / 125 (70 / 239 / 951), 1024 x 3072 35 / 41 / 133
+// (100 / 370 / 1469).
+int launch_rows_group(int M, int N, int K, const uint8_t* const* w, const uint16_t* const* s, const void* const* x,
+                      void* const* y, int count, bool xf32, int xp, int ep, hipStream_t st) {
+  if (count <= 0 || !xp || (ep != EP_F16 && ep != EP_F32)) return Q4D_ERR_SHAPE;
+  for (int i = 0; i < count; ++i)
+    if (const int rc = check_rows(RowsArgs{w[i], s[i], x[i], y[i], nullptr, M, N, K}, xf32, xp, ep)) return rc;
+  for (int i0 = 0; i0 < count; i0 += kRowsGroupMax) {
+    const int n = count - i0 < kRowsGroupMax ? count - i0 : kRowsGroupMax;
+    int rc;
+    if (n == 1) {
+      rc = launch_rows(RowsArgs{w[i0], s[i0], x[i0], y[i0], nullptr, M, N, K}, xf32, xp, ep, st);
+    } else {
+      RowsGroupArgs g;
+      g.a = RowsArgs{nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K};
+      for (int k = 0; k < kRowsGroupMax; ++k) {
+        const int i = i0 + (k < n ? k : 0);  // unused slots repeat the first matrix, never read
+        g.w[k] = w[i];
+        g.s[k] = s[i];
+        g.x[k] = x[i];
+        g.y[k] = y[i];
+      }
+      const bool f16 = ep == EP_F16;
+      if (xf32 && xp == 2)
+        rc = f16 ? launch_group_nt<true, 2, EP_F16>(g, n, st) : launch_group_nt<true, 2, EP_F32>(g, n, st);
+      else if (xf32)
+        rc = f16 ? launch_group_nt<true, 1, EP_F16>(g, n, st) : launch_group_nt<true, 1, EP_F32>(g, n, st);
+      else
+        rc = f16 ? launch_group_nt<false, 1, EP_F16>(g, n, st) : launch_group_nt<false, 1, EP_F32>(g, n, st);
+    }
+    if (rc) return rc;
+  }
+  return Q4D_OK;
 }
 
 }  // namespace q4d

@@ -11,6 +11,7 @@ import oracle as o
 from gpu_helpers import linear, q4
 from llm_accelerator_amd import _lib
 from llm_accelerator_amd._lib import Q4D_F16, Q4D_F32
+from llm_accelerator_amd.model import Q4Tensor
 
 pytestmark = pytest.mark.gpu
 
@@ -94,6 +95,52 @@ def test_linear_group_rows_equal_single_calls(dev):
                "q4d_linear_group")
     for w, x, y in zip(ws, xs, ys):
         assert torch.equal(y, linear(w, x))
+
+
+@pytest.mark.parametrize("m,n,k,count,xdtype,ydtype,precision", [
+    (4, 130, 1024, 70, torch.float32, Q4D_F32, 2),      # launches of 64 + 6, each block one tile
+    (5, 1026, 3072, 64, torch.float32, Q4D_F16, 2),     # four weight tiles per block, the waves of one
+    (20, 66, 3072, 2, torch.float32, Q4D_F32, 2),       # one tile, 12 waves
+    (33, 3072, 3072, 3, torch.float32, Q4D_F32, 2),     # two weight tiles alone, two row tiles together
+    (40, 512, 2048, 65, torch.float16, Q4D_F16, 1),     # 64 + 1: the last a launch of its own
+    (17, 512, 3072, 66, torch.float32, Q4D_F32, 1),
+    (64, 258, 1024, 30, torch.float16, Q4D_F32, 1),
+    (70, 130, 2048, 64, torch.float32, Q4D_F32, 2),     # two row tiles, the general loop
+])
+def test_linear_group_rows_one_launch_and_bits(dev, m, n, k, count, xdtype, ydtype, precision):
+    """q4d_linear_group at 4 rows and more: one launch per 64 matrices (the kernels a captured call
+    records), and each output equals its own q4d_linear call bit for bit whatever tile the group takes."""
+    from llm_accelerator_amd.model import current_stream
+    lib = _lib.load()
+    g = torch.Generator(device=dev).manual_seed(m + n + k)
+    mats = [Q4Tensor(torch.randint(0, 256, (n, k // 2), generator=g, device=dev, dtype=torch.uint8),
+                     torch.randint(1, 3000, (n, k // 64), generator=g, device=dev).to(torch.int16).view(torch.uint16))
+            for _ in range(count)]
+    xs = [torch.randn(m, k, generator=g, device=dev).to(xdtype) for _ in range(count)]
+    ydt = torch.float16 if ydtype == Q4D_F16 else torch.float32
+    ys = [torch.full((m, n), float("nan"), device=dev, dtype=ydt) for _ in range(count)]
+    descs = (_lib.Q4dMatrix * count)(*[w.descriptor() for w in mats])
+    xp, yp = ((ctypes.c_void_p * count)(*[t.data_ptr() for t in ts]) for ts in (xs, ys))
+    xcode = Q4D_F16 if xdtype == torch.float16 else Q4D_F32
+    print(f"[linear group rows] {count} x {m} x {n} x {k}", flush=True)
+
+    def call():
+        _lib.check(lib.q4d_linear_group(descs, xp, xcode, yp, ydtype, m, count, current_stream()), "q4d_linear_group")
+
+    _lib.check(lib.q4d_set_activation_precision(precision), "q4d_set_activation_precision")
+    try:
+        call()
+        for w, x, y in zip(mats, xs, ys):
+            assert torch.equal(y, linear(w, x, ydtype))
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph):
+            call()
+    finally:
+        _lib.check(lib.q4d_set_activation_precision(2), "q4d_set_activation_precision")
+    nodes = ctypes.c_size_t(0)
+    lib.hipGraphGetNodes.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_size_t)]
+    assert lib.hipGraphGetNodes(graph.raw_cuda_graph(), None, ctypes.byref(nodes)) == 0
+    assert nodes.value == (count + 63) // 64
 
 
 @pytest.mark.parametrize("m,n,k,top", [(1, 128, 1024, 1500), (33, 1024, 3072, 1500), (64, 384, 2048, 9000),
