@@ -314,7 +314,8 @@ int launch_group_nt(const RowsGroupArgs& g, int count, hipStream_t st) {
 
 // The largest tile (each split activation serves NT weight tiles, each unpacked weight MT row
 // tiles) that still gives most CUs a block: 512 rows of 3072 x 1024, fp16: 24.4 us with
-// MT = 1, 16.3 with 2; 64 rows of 2048 x 1024: 3.6 us on 256 blocks, 4.8 on 128.
+// MT = 1, 16.3 with 2; 64 rows of 2048 x 1024: 3.6 us on 256 blocks, 4.8 on 128.  Two row
+// tiles only where there are two: 4 fp32 rows of 151936 x 1024 27.5 us, 48.4 with MT = 2.
 // One matrix of K = 3072 on one-tile blocks: 12 waves of two units (4 rows: 5.1 us, 5.5 with 8
 // of three), which groups the sums differently from 8 waves.  The matrices of a group count
 // together, but each keeps its own launch's waves, so its bits are its own launch's (12 waves
@@ -324,7 +325,7 @@ RowsTile rows_tile(int M, int N, int K, int count) {
   const auto blocks = [&](int m, int n) { return (long)((mt + m - 1) / m) * ((nt + n - 1) / n); };
   constexpr long kMinBlocks = 192;
   RowsTile t = {1, 1, false};
-  if (blocks(2, 4) >= kMinBlocks) t = {2, 4, false};
+  if (mt > 1 && blocks(2, 4) >= kMinBlocks) t = {2, 4, false};
   else if (blocks(1, 4) >= kMinBlocks) t = {1, 4, false};
   else if (blocks(1, 2) >= kMinBlocks) t = {1, 2, false};
   else t.k12 = K == 24 * kRwUnit;
