@@ -213,7 +213,7 @@ bool chain_applies(const GemmArgs& a, int ep, bool pair) {
     if (!aligned(a.s[i], 4)) return false;
   if (ep == EP_ROPE || ep == EP_SWIGLU)
     return a.K == 1024 && !a.part && a.ksplit <= 1 && (ep == EP_ROPE || (a.ldy % 2 == 0 && aligned(a.y, 4)));
-  if (ep != EP_RESID || a.nseg != 1 || a.ksplit < 1 || !a.part || !aligned(a.part, 16) ||
+  if (ep != EP_RESID || a.nseg != 1 || a.ksplit < 2 || !a.part || !aligned(a.part, 16) ||
       (size_t)a.ksplit * a.M * a.N > a.part_cap || a.K % a.ksplit)
     return false;
   const int ks = a.K / a.ksplit;

@@ -387,7 +387,7 @@ struct GemmArgs {
   PrefillArgs rope;
 };
 // The prefill GEMMs of short prompts (q4d_chain.hip): EP_ROPE and EP_SWIGLU without a split,
-// EP_RESID with a.ksplit splits into a.part (raw partial tiles; the reduction is the caller's).
+// EP_RESID with a.ksplit >= 2 splits into a.part (raw partial tiles; the reduction is the caller's).
 bool chain_applies(const GemmArgs& a, int ep, bool pair);
 int launch_chain(const GemmArgs& a, int ep, bool pair, hipStream_t st);
 constexpr int kGemmMaxSplit = 16;

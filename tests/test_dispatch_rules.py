@@ -24,6 +24,17 @@ int main() {
       if (scanf("%d %d %d %d", &M, &N, &K, &count) != 4) return 1;
       const RowsTile t = rows_tile(M, N, K, count);
       printf("%d %d %d\n", t.mt, t.nt, (int)t.k12);
+    } else if (!strcmp(rule, "chain_resid")) {  // an output projection of a short prefill
+      GemmArgs a;
+      memset(&a, 0, sizeof(a));
+      if (scanf("%d %d %d %d", &a.M, &a.N, &a.K, &a.ksplit) != 4) return 1;
+      static float memory[64];  // aligned; never read
+      a.nseg = 1;
+      a.seg_end[0] = a.N;
+      a.s[0] = (const uint16_t*)align_up((size_t)memory, 16);
+      a.part = (float*)align_up((size_t)memory, 16);
+      a.part_cap = (size_t)1 << 40;
+      printf("%d\n", (int)chain_applies(a, EP_RESID, false));
     } else {
       return 1;
     }
@@ -65,3 +76,12 @@ def test_rows_tile_has_no_tile_of_padding_rows(rule, k, count):
         if count > 1:
             assert mt == 1 or not k12
             assert nt in (1, 4), (m, n)   # the tiles that the grouped kernel has
+
+
+def test_chain_resid_needs_a_split(rule):
+    """The short prefill's output projections write raw partial tiles, which a reduction adds: without a
+    split there is none, so y would never be written."""
+    cases = [(m, n, k, ksplit) for m in (1, 75, 512) for n, k in ((1024, 512), (1024, 1024), (1024, 1536),
+                                                                  (1024, 2048), (1024, 3072)) for ksplit in (0, 1, 2)]
+    for c, (applies,) in zip(cases, rule([("chain_resid", *c) for c in cases])):
+        assert applies == (c[3] == 2 and c[2] // 2 in (512, 1024, 1536)), c
