@@ -1054,7 +1054,7 @@ int q4d_rotate_half(const float* x, float* y, int64_t rows, int32_t head_dim, vo
 
 size_t q4d_causal_attention_workspace_bytes(int32_t batch, int32_t q_heads, int32_t kv_heads, int32_t seq) {
   if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || seq <= 0) return 0;
-  return causal_attention_ws_bytes(batch, q_heads, kv_heads, seq);
+  return causal_attention_ws_bytes(batch, kv_heads, seq);
 }
 
 int q4d_causal_attention(const float* q, const float* k, const float* v, float* out, int32_t batch,
@@ -1067,7 +1067,7 @@ int q4d_causal_attention(const float* q, const float* k, const float* v, float* 
   if ((long long)batch * q_heads * seq * head_dim > (1LL << 40)) return Q4D_ERR_SHAPE;
   if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 16) || !aligned(ws, 256))
     return Q4D_ERR_BAD_ADDR;
-  if (ws_bytes < causal_attention_ws_bytes(batch, q_heads, kv_heads, seq)) return Q4D_ERR_CAPACITY;
+  if (ws_bytes < causal_attention_ws_bytes(batch, kv_heads, seq)) return Q4D_ERR_CAPACITY;
   return launch_causal_attention(q, k, v, out, batch, q_heads, kv_heads, seq, scaling, ws, as_stream(stream));
 }
 

@@ -476,8 +476,8 @@ int launch_apply_rope(const float* x, float* y, const float* cosv, const float* 
 int launch_rotate_half(const float* x, float* y, long long rows, int head_dim, hipStream_t stream);
 // Causal GQA attention over fp32 q [batch, qh, seq, 128], k / v [batch, kvh, seq, 128]
 // -> fp32 out [batch, qh, seq, 128] through prefill_attn_kernel (q4d_prefill.hip);
-// ws holds the fp16 operands (causal_attention_ws_bytes).
-size_t causal_attention_ws_bytes(int batch, int qh, int kvh, int seq);
+// ws holds k and v as fp16 (causal_attention_ws_bytes).
+size_t causal_attention_ws_bytes(int batch, int kvh, int seq);
 int launch_causal_attention(const float* q, const float* k, const float* v, float* out, int batch, int qh,
                             int kvh, int seq, float scaling, void* ws, hipStream_t st);
 

@@ -349,19 +349,15 @@ __global__ __launch_bounds__(256) void kv_to_f16_kernel(const float* k, const fl
 
 }  // namespace
 
-size_t causal_attention_ws_bytes(int batch, int qh, int kvh, int seq) {
-  const size_t A = 256;
-  const size_t q = align_up((size_t)batch * qh * seq * kD * 2, A);
-  const size_t kv = align_up((size_t)batch * kvh * seq * kD * 2, A);
-  const size_t o = align_up((size_t)seq * qh * kD * 2, A);
-  return q + 2 * kv + o;
+size_t causal_attention_ws_bytes(int batch, int kvh, int seq) {
+  return 2 * align_up((size_t)batch * kvh * seq * kD * 2, 256);  // the fp16 k and v planes
 }
 
 int launch_causal_attention(const float* q, const float* k, const float* v, float* out, int batch, int qh,
                             int kvh, int seq, float scaling, void* ws, hipStream_t st) {
   const size_t kvn = (size_t)batch * kvh * seq * kD;
   _Float16* k16 = static_cast<_Float16*>(ws);
-  _Float16* v16 = reinterpret_cast<_Float16*>(static_cast<char*>(ws) + align_up(kvn * 2, 256));
+  _Float16* v16 = reinterpret_cast<_Float16*>(static_cast<char*>(ws) + causal_attention_ws_bytes(batch, kvh, seq) / 2);
   const long long n8 = (long long)(kvn / 8), blocks = (n8 + 255) / 256;
   hipLaunchKernelGGL(kv_to_f16_kernel, dim3((unsigned)(blocks < 8192 ? blocks : 8192), 2), dim3(256), 0, st, k, v, k16,
                      v16, n8);

@@ -319,3 +319,13 @@ def test_linear_group_checks_every_matrix_before_the_first_launch(lib):
     assert f(mats, ptrs, 1, ys, 1, 1, n, None) == -7            # y[69]
     xs = (ctypes.c_void_p * n)(*([FAKE] * (n - 1) + [FAKE + 8]))
     assert f(mats, xs, 1, ptrs, 1, 1, n, None) == -4            # x[69] alignment
+
+
+@pytest.mark.parametrize("b,qh,kvh,s", [(1, 16, 8, 1), (2, 16, 8, 1500), (3, 3, 3, 37), (1, 32, 1, 100)])
+def test_causal_attention_workspace_is_the_fp16_k_and_v(lib, b, qh, kvh, s):
+    """The prompt attention keeps k and v as fp16 planes and reads q and writes the output in fp32 where
+    they are: no more scratch than those planes, and a byte less is refused before any launch."""
+    plane = -(-(b * kvh * s * 128 * 2) // 256) * 256
+    need = lib.q4d_causal_attention_workspace_bytes(b, qh, kvh, s)
+    assert need == 2 * plane
+    assert lib.q4d_causal_attention(FAKE, FAKE, FAKE, FAKE, b, qh, kvh, s, 128, 0.1, FAKE, need - 1, None) == -9

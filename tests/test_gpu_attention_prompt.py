@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 import torch
 
-from llm_accelerator_amd import common
+from llm_accelerator_amd import _lib, common
+from llm_accelerator_amd.model import current_stream
 
 pytestmark = pytest.mark.gpu
 
@@ -40,6 +41,24 @@ def test_prompt_attention_vs_fp64(dev, b, h, kvh, s):
     # probabilities rounded to fp16 against a maximum up to 2^8 below theirs (2^-11 each),
     # fp32 scores (exponent error 2^-22 of |score| <= 2^12, times ln 2)
     assert torch.all((out.double() - ref).abs() <= 2.0 ** -9 * size + 1e-6)
+
+
+@pytest.mark.parametrize("b,h,kvh,s", [(1, 16, 8, 1), (3, 16, 8, 67), (2, 5, 1, 130)])
+def test_prompt_attention_stays_in_its_workspace(dev, b, h, kvh, s):
+    """A workspace of exactly the stated bytes between two guards: the guards stay, and the output is
+    that of a call with room to spare."""
+    lib = _lib.load()
+    q, k, v = (torch.randn(b, n, s, 128, device=dev) for n in (h, kvh, kvh))
+    need = int(lib.q4d_causal_attention_workspace_bytes(b, h, kvh, s))
+    outs = []
+    for nbytes in (need, 4 * need + 4096):
+        ws = torch.full((256 + nbytes + 4096,), 0x5A, dtype=torch.uint8, device=dev)
+        out = torch.full_like(q, float("nan"))
+        _lib.check(lib.q4d_causal_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, kvh, s, 128,
+                                            0.09, ws.data_ptr() + 256, nbytes, current_stream()), "q4d_causal_attention")
+        outs.append(out)
+        assert bool((ws[:256] == 0x5A).all()) and bool((ws[256 + need:] == 0x5A).all())
+    assert torch.equal(*outs) and bool(torch.isfinite(outs[0]).all())
 
 
 def test_prompt_attention_sequences_are_independent(dev):
