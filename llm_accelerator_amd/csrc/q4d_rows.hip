@@ -273,23 +273,33 @@ int launch_tile(const Args& args, const RowsArgs& a, int count, bool k12, hipStr
   const dim3 grid((a.N + 16 * NT - 1) / (16 * NT), (a.M + 16 * MT - 1) / (16 * MT), count);
   const auto go = [&](auto kernel, int nw) { hipLaunchKernelGGL(kernel, grid, dim3(64 * nw), 0, st, args); };
   // Every unit of a wave in flight where K is one of the projections' widths and the
-  // registers hold them (211 x 1024 x 3072, hi + lo: 9.5 us, 11.5 with the next unit only).
+  // registers hold them (211 x 1024 x 3072, hi + lo: 8.6 us, 11.5 with the next unit only);
+  // else the general loop, which q4d_linear needs for one tile and q4d_gemm for other widths.
   constexpr bool kDeep = XP < 2 || MT * NT <= 4, kGroup = std::is_same_v<Args, RowsGroupArgs>;
   constexpr bool k12Tile = MT == 1 && (NT == 1 || kGroup);  // the tiles that rows_tile gives 12 waves
-  const int nu = a.K / kRwUnit;
-  if constexpr (k12Tile)
-    if (nu == 24 && k12) {
-      go(rows_kernel<XF32, XP, EP, MT, NT, 12, 2, Args>, 12);
-      return check_launch();
-    }
-  if (nu == 8)
-    go(rows_kernel<XF32, XP, EP, MT, NT, 8, 1, Args>, 8);
-  else if (nu == 16 && kDeep)
-    go(rows_kernel<XF32, XP, EP, MT, NT, 8, kDeep ? 2 : 0, Args>, 8);
-  else if (nu == 24 && kDeep && NT > 1)
-    go(rows_kernel<XF32, XP, EP, MT, NT, 8, (kDeep && NT > 1) ? 3 : 0, Args>, 8);
-  else
-    go(rows_kernel<XF32, XP, EP, MT, NT, 8, 0, Args>, 8);
+  switch (a.K / kRwUnit) {
+    case 8: go(rows_kernel<XF32, XP, EP, MT, NT, 8, 1, Args>, 8); return check_launch();
+    case 16:
+      if constexpr (kDeep) {
+        go(rows_kernel<XF32, XP, EP, MT, NT, 8, 2, Args>, 8);
+        return check_launch();
+      }
+      break;
+    case 24:
+      if constexpr (k12Tile)
+        if (k12) {
+          go(rows_kernel<XF32, XP, EP, MT, NT, 12, 2, Args>, 12);
+          return check_launch();
+        }
+      if constexpr (kDeep && NT > 1) {
+        go(rows_kernel<XF32, XP, EP, MT, NT, 8, 3, Args>, 8);
+        return check_launch();
+      }
+      break;
+    default: break;
+  }
+  if constexpr (XP != 0 && kDeep) return Q4D_ERR_SHAPE;  // q4d_linear's widths are above
+  else go(rows_kernel<XF32, XP, EP, MT, NT, 8, 0, Args>, 8);
   return check_launch();
 }
 
