@@ -90,12 +90,12 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const Args args) {
 #pragma unroll
   for (int i = 0; i < XR; ++i) xo[i] = (uint32_t)min(4 * i + xr, a.M - 1 - m0) * a.K * XB + 8 * XB * xc;
 
-  // where a lane stores them in LDS.  Other lanes of the wave read them: its LDS operations run
-  // in program order, and the empty asm holds the compiler to that order, since it cannot tell
-  // an opaque offset apart from any load's.  (A wave barrier with fences does too, but stops
-  // the scheduler: 211 fp32 rows of 1024 x 3072 8.6 -> 9.4 us.)
-  uint32_t xw = xr * kRwLd + 8 * xc;
-  asm("" : "+v"(xw));
+  // where the wave stores them in LDS.  Other lanes of the wave read them: its LDS operations
+  // run in program order, and the empty asm holds the compiler to that order, since it cannot
+  // tell an opaque offset apart from any load's.  (A wave barrier with fences does too, but
+  // stops the scheduler: 211 fp32 rows of 1024 x 3072 8.6 -> 9.4 us.)
+  uint32_t xw = (uint32_t)w * kH * 16 * MT * kRwLd;
+  asm("" : "+s"(xw));
 
   struct Unit {
     u32x4 x[XL];
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(const Args args) {
     // activations to LDS in pair order: row 4 i + xr, hi at 0, lo 16 MT rows further
 #pragma unroll
     for (int i = 0; i < XR; ++i) {
-      u32x4* d = reinterpret_cast<u32x4*>(xs + xw + 4 * i * kRwLd);
+      u32x4* d = reinterpret_cast<u32x4*>(reinterpret_cast<_Float16*>(lds) + xw + (4 * i + xr) * kRwLd + 8 * xc);
       if constexpr (XF32) {
         u32x4 hw, lw;
 #pragma unroll
