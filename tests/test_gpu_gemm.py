@@ -171,8 +171,9 @@ def test_gemm_splitk_integer_exact(dev, N, K, M, ksplit):
 def test_gemm_many_rows_splitk_integer_exact(dev, N, K, M, ksplit):
     """Split-K at prefill-sized M with the residual epilogue: the prefill down shape
     (N = 1024, K = 3072, M = 2048) with a 2-way split runs the pipelined kernel
-    (128 tiles x 2 splits fill the device in one round), 4-way and automatic splits
-    the 128-row-tile kernel; M = 300 ends on a partial row tile."""
+    (128 tiles x 2 splits fill the device in one round), automatically without a split,
+    and 4-way the 64-row tiles; M = 300 ends on a partial row tile (2-way pipelined,
+    4-way 64-row tiles, automatically the rows kernel)."""
     rng = np.random.default_rng(N + K + M + ksplit)
     packed, scale, x, ref = exact_case(rng, N, K, M)
     print(f"[gemm splitk many rows] M={M} N={N} K={K} ksplit={ksplit}", flush=True)
