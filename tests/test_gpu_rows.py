@@ -98,7 +98,7 @@ def test_linear_group_rows_equal_single_calls(dev):
 
 
 @pytest.mark.parametrize("m,n,k,count,xdtype,ydtype,precision", [
-    (4, 130, 1024, 70, torch.float32, Q4D_F32, 2),      # launches of 64 + 6, each block one tile
+    (4, 130, 1024, 70, torch.float32, Q4D_F32, 2),      # 64 + 6: four weight tiles per block, then one
     (5, 1026, 3072, 64, torch.float32, Q4D_F16, 2),     # four weight tiles per block, the waves of one
     (20, 66, 3072, 2, torch.float32, Q4D_F32, 2),       # one tile, 12 waves
     (33, 3072, 3072, 3, torch.float32, Q4D_F32, 2),     # two weight tiles alone, two row tiles together
@@ -145,11 +145,13 @@ def test_linear_group_rows_one_launch_and_bits(dev, m, n, k, count, xdtype, ydty
 
 @pytest.mark.parametrize("m,n,k,top", [(1, 128, 1024, 1500), (33, 1024, 3072, 1500), (64, 384, 2048, 9000),
                                        (100, 3072, 1024, 4095), (500, 3072, 1024, 1500), (401, 1024, 3072, 1500),
-                                       (64, 128, 1152, 65535), (700, 4096, 1024, 9000), (2000, 1024, 2048, 9000)])
+                                       (64, 128, 1152, 65535), (700, 4096, 1024, 9000), (2000, 1024, 2048, 9000),
+                                       (2000, 4096, 1024, 9000)])
 def test_gemm_vs_fp16_operands(dev, m, n, k, top):
     """q4d_gemm against the product of the same fp16 operands (weights rounded once): the rows
-    kernel's tile sizes and general K loop (1152 columns), the tiled and the pipelined kernel,
-    with scale codes on both sides of the fast conversion's limit (4094)."""
+    kernel's tile sizes and general K loop (1152 columns), the pipelined kernel (700 x 4096, 2000 x
+    1024) and the 128-row tiles (2000 x 4096), with scale codes on both sides of the fast
+    conversion's limit (4094)."""
     from llm_accelerator_amd.model import current_stream
     rng = np.random.default_rng(m + n + k)
     packed = rng.integers(0, 256, size=(n, k // 2), dtype=np.uint8)
