@@ -424,43 +424,73 @@ __device__ __forceinline__ int wave_scan(int x) {
 constexpr int kSpanSplits = 16;  // splits of one sequence at most
 constexpr int kSpanMerge = 8;    // splits merged in one batch of loads
 
-// Which part of which sequence block `idx` of a kv head takes.
-struct SpanWork {
-  int b, s, nsplit, pos;  // b < 0: none
+// The cut of a batch's sequences into parts; one block takes one part for one kv head.  A CU
+// works on one block about as fast as on two (24 x 1024 positions in 192 / 384 / 576 blocks:
+// 19.8 / 21.4 / 23.5 us), so the parts number at most one block per CU, or two where the
+// sequences alone are more than one: `slots` parts per kv head.  With S = all sub-chunks / slots
+// a sequence of n sub-chunks takes floor(n / S + up) parts, at least one.  up rounds a long
+// sequence of a ragged batch up (24 x 649-1500 positions 24.4 -> 23.5 us) where that does not
+// cut every sequence of an equal batch once more (12 x 1024: 13.0 us in 24 parts, 15.4 in 36).
+//
+// A split costs ~2 us (partials, count-in, merge) and a sub-chunk ~0.85, so it has to shorten
+// the sequence by three sub-chunks: 24 x 100 positions 4.9 us whole, 7.1 in two parts.  Past
+// eight sub-chunks a part has two or more, and more than eight parts, a second batch of merge
+// loads, have four or more.  Since up <= 1/2 the parts past the sequences' first number at most
+// `slots`, which is what the grid holds.  A position out of range is one part of no sub-chunks.
+struct SpanRule {
+  float slots, up;
+  float slots_long, up_long;  // the same from kSpanLong sub-chunks a sequence on
+  int cut;                    // 0: one part per sequence
+};
+constexpr int kSpanLong = 40;
+
+struct SpanCut {
+  float inv, up;  // 1 / S
 };
 
-// Every sequence is cut into round(its sub-chunks / S) parts, at least one, with
-// S = ceil(all sub-chunks / slots): the parts number at most slots + batch, which is the
-// launcher's grid.  Rounded up, the sequences a little longer than S became two short parts
-// and a merge (64 x 285-600 positions: 23.9 us, 21.4 as one part each).  More than eight
-// parts of one sequence cost a second batch of merge loads, so they have four sub-chunks or
-// more each.  Batches of `slots` sequences and more are one part per sequence, without the
-// cut's ~0.4 us (64 sequences: equal lengths 43.2 against 43.6 us, 47-2000 positions 48.1
-// against 49.4).  A position out of range counts as one part of no sub-chunks, whose
-// block reports it.  Every wave of every block computes the same split from the positions
-// (lane l: sequence g + l).
-__device__ __forceinline__ SpanWork span_work(const AttnArgs& a, int idx, int slots, int lane) {
-  if (a.batch >= slots) return {idx, 0, 1, a.positions[idx]};
-  const auto load = [&](int b) { return b < a.batch ? a.positions[b] : -1; };
-  const auto subs = [&](int p) { return p >= 0 && p < a.max_ctx ? p / kAttnChunk + 1 : 0; };
-  int p = load(lane);
-  int total = __builtin_amdgcn_readlane(wave_scan(subs(p)), 63);
-  for (int g = kWave; g < a.batch; g += kWave) total += __builtin_amdgcn_readlane(wave_scan(subs(load(g + lane))), 63);
-  const int S = max(1, (total + slots - 1) / slots);
+__device__ __forceinline__ int span_subs(const AttnArgs& a, int p) {
+  return p >= 0 && p < a.max_ctx ? p / kAttnChunk + 1 : 0;
+}
+
+// Parts of a sequence of n sub-chunks.
+__device__ __forceinline__ int span_parts(int n, const SpanCut& c) {
+  const int most = n > 8 ? max(min(kSpanMerge, (n + 1) >> 1), min(kSpanSplits, n >> 2)) : 8;
+  const int q = min((int)fmaf((float)n, c.inv, c.up), most);
+  return q > 1 && n >= max(4, 8 - q) ? q : 1;  // n - ceil(n / q) >= 3
+}
+
+// Every wave of every block computes the same cut.  p: the position of sequence `lane`, -1 past
+// the batch.
+__device__ __forceinline__ SpanCut span_cut(const AttnArgs& a, int p, const SpanRule& r, int lane) {
+  int total = __builtin_amdgcn_readlane(wave_scan(span_subs(a, p)), 63);
+  for (int g = kWave; g < a.batch; g += kWave) {
+    const int q = g + lane < a.batch ? a.positions[g + lane] : -1;
+    total += __builtin_amdgcn_readlane(wave_scan(span_subs(a, q)), 63);
+  }
+  const bool lg = total >= kSpanLong * a.batch;
+  return {fminf(1.f, (lg ? r.slots_long : r.slots) * __builtin_amdgcn_rcpf((float)total)), lg ? r.up_long : r.up};
+}
+
+// Which part of which sequence extra block `idx` of a kv head takes: the sequences' parts past
+// their first, in order.  b < 0: none.
+struct SpanWork {
+  int b, s, nsplit, pos;
+};
+
+__device__ __forceinline__ SpanWork span_extra(const AttnArgs& a, int idx, const SpanCut& c, int p, int lane) {
   for (int g = 0;;) {
-    const int n0 = subs(p), most = max(kSpanMerge, min(kSpanSplits, n0 / 4));
-    const int ns = g + lane < a.batch ? min(most, max(1, (n0 + S / 2) / S)) : 0;
+    const int ns = span_parts(span_subs(a, p), c) - 1;
     const int incl = wave_scan(ns);
     const int all = __builtin_amdgcn_readlane(incl, 63);
     if (idx < all) {
       const int l = __builtin_ctzll(__ballot(incl > idx));
       const int n = __builtin_amdgcn_readlane(ns, l);
-      return {g + l, idx - __builtin_amdgcn_readlane(incl, l) + n, n, __builtin_amdgcn_readlane(p, l)};
+      return {g + l, idx - __builtin_amdgcn_readlane(incl, l) + n + 1, n + 1, __builtin_amdgcn_readlane(p, l)};
     }
     idx -= all;
     g += kWave;
     if (g >= a.batch) return {-1, 0, 0, 0};
-    p = load(g + lane);
+    p = g + lane < a.batch ? a.positions[g + lane] : -1;
   }
 }
 
@@ -472,38 +502,45 @@ __device__ __forceinline__ SpanWork span_work(const AttnArgs& a, int idx, int sl
 // and sum L per head; its output accumulators are rescaled by 2^(M_old - M_new)
 // when M grows) over its 16 positions of every sub-chunk, so the sub-chunk loop has
 // no barrier; the four waves' states are merged once after the span.  K/V are read
-// with non-temporal loads (read once per step).  The parts are cut from the
-// sequences' own positions (span_work) to about two blocks per CU of nearly equal
-// length: a few long contiguous K/V streams per CU read HBM faster than many short
-// ones (64 x 4097 positions, 28 layers: eight 576-position spans per head, 5
-// resident blocks per CU and 32-position sub-chunks took 6.35 ms per step; equal
+// with non-temporal loads (read once per step): a few long contiguous K/V streams per CU read
+// HBM faster than many short ones (64 x 4097 positions, 28 layers: eight 576-position spans
+// per head, 5 resident blocks per CU and 32-position sub-chunks took 6.35 ms per step; equal
 // parts 6.27; one block per head with 64-position sub-chunks 5.48).
-// Cut from the capacity instead, as before, one long part held up ragged batches and short
-// contexts of a large cache ran on few blocks (us a call, before / now): 24 x 649-1500
-// positions 24.8 / 21.8, 8 x 2000 of 8192 31.0 / 17.8, 40 x 660-3000 of 4096 63.6 / 55.8, one
-// sequence of 8000 18.4 / 13.4; uniform batches that fill the cache within 2 %.
+// The parts are cut from the sequences' own positions (SpanRule).  Cut from the capacity
+// instead, one long part held up ragged batches and short contexts of a large cache ran on few
+// blocks (us a call, from the capacity / now): 24 x 649-1500 positions of 2048 25.9 / 23.5, 8 x
+// 2048 of 8192 31.7 / 14.5, 40 x 2048 of 4096 79 / 62, one sequence of 8191 18.7 / 14.1; equal
+// batches that fill the cache are within 3 % (one of 952 of 1024 6.8 / 7.1), 24 x 4095 of 4096
+// 75 / 64.  The first parts' loads go out before the cut is known, which hides its ~0.4 us from
+// the sequences that stay whole.
 // Same prologue and partial format as attn_kernel<64>; thread t owns dims
 // 8 (t % 16) .. +7 of positions t / 16 + 16 i.
-__global__ __launch_bounds__(256) void attn_span_kernel(const AttnArgs a, int slots) {
+__global__ __launch_bounds__(256) void attn_span_kernel(const AttnArgs a, const SpanRule rule) {
   attn_preload(a);
   constexpr int D = 128, CH = kAttnChunk, NPT = CH / 16;
   const int t = threadIdx.x, lane = t & 63;
   const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
   const int idx = blockIdx.x / a.kvh, j = blockIdx.x - idx * a.kvh;
-  const SpanWork wk = span_work(a, idx, slots, lane);
-  const int b = wk.b, s = wk.s, nsplit = wk.nsplit, pos = wk.pos;
-  if (b < 0) return;
+  // the first `batch` blocks of a kv head are the sequences' first parts: their loads go out
+  // before the cut is known
+  const bool first = idx < a.batch;
+  const int lpos = rule.cut && lane < a.batch ? a.positions[lane] : -1;
+  int b = idx, s = 0, nsplit = 1, pos;
+  if (first) {
+    pos = a.positions[idx];
+  } else {
+    const SpanWork wk = span_extra(a, idx - a.batch, span_cut(a, lpos, rule, lane), lpos, lane);
+    if (wk.b < 0) return;
+    b = wk.b; s = wk.s; nsplit = wk.nsplit; pos = wk.pos;
+  }
   if (pos < 0 || pos >= a.max_ctx) {
     if (j == 0 && t == 0) atomicOr(a.status, Q4D_STATUS_BAD_POSITION);
     return;
   }
   const int T = pos + 1;
   const int nsub_all = (T + CH - 1) / CH;
-  const int start = (s * nsub_all / nsplit) * CH;
-  const int end = min(T, ((s + 1) * nsub_all / nsplit) * CH);
-  const int nsub = (end - start + CH - 1) / CH;
+  const int start = first ? 0 : (s * nsub_all / nsplit) * CH;
   const int cached = a.fused ? pos : T;
-  const bool last = (s == nsplit - 1);  // block-uniform: holds pos
 
   __shared__ float sq[2][D];
   __shared__ uint16_t snew[2][D];
@@ -518,8 +555,6 @@ __global__ __launch_bounds__(256) void attn_span_kernel(const AttnArgs a, int sl
   // ---- q / new k / new v rows first (as attn_kernel) ----------------------------
   const float qscale = a.scaling * 1.4426950408889634f;
   const int qkv_stride = (a.qh + 2 * a.kvh) * D;
-  const bool qk_wave = a.fused ? (wid < 2 || (last && wid == 2)) : (wid < 2);
-  const bool v_wave = a.fused && last && wid == 3;
   const float* row;
   const float* gam;
   const float* ctab;
@@ -552,6 +587,16 @@ __global__ __launch_bounds__(256) void attn_span_kernel(const AttnArgs a, int sl
     kr[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kb + (size_t)p * D + sub * 8));
     vr[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vb + (size_t)p * D + sub * 8));
   }
+
+  __builtin_amdgcn_sched_barrier(0);
+
+  // the rest of the part, once its loads are out
+  if (first && rule.cut && nsub_all >= 4) nsplit = span_parts(nsub_all, span_cut(a, lpos, rule, lane));
+  const int end = min(T, ((s + 1) * nsub_all / nsplit) * CH);
+  const int nsub = (end - start + CH - 1) / CH;
+  const bool last = (s == nsplit - 1);  // block-uniform: holds pos
+  const bool qk_wave = a.fused ? (wid < 2 || (last && wid == 2)) : (wid < 2);
+  const bool v_wave = a.fused && last && wid == 3;
 
   // ---- per-head RMSNorm (common.py:258-262) + rotate-half RoPE (264-268) -------
   if (a.fused && qk_wave) {
@@ -769,16 +814,24 @@ int launch_attention(const AttnArgs& a, hipStream_t stream) {
   if (!a.part_ml || !a.part_acc || (a.merge && !a.counters)) return Q4D_ERR_NULL;
   if (a.merge) {
     // contexts past 512 positions: the sequences' positions are on the device, so the
-    // grid is the bound of span_work's parts and blocks past the last part end at once
+    // grid is the bound of the cut's parts and blocks past the last part end at once
     const int nch = (a.max_ctx + kAttnChunk - 1) / kAttnChunk;
     if (nch <= kSpanMerge) {
       hipLaunchKernelGGL(attn_kernel<kAttnChunk>, dim3(a.nsplit_max, a.kvh, a.batch), dim3(256), 0, stream, a);
     } else {
-      const int slots = max(1, 2 * device_cus() / a.kvh);
-      const long long parts = a.batch >= slots
-                                  ? a.batch
-                                  : min((long long)a.batch * min(kSpanSplits, nch), (long long)a.batch + slots);
-      hipLaunchKernelGGL(attn_span_kernel, dim3((unsigned)(parts * a.kvh)), dim3(256), 0, stream, a, slots);
+      const int per = max(1, device_cus() / a.kvh);
+      // past one block per CU, long sequences fill the last round's CUs (36 / 40 x 3072 positions
+      // 89 / 90 us whole, 83 / 86 in two parts each; 48 x 3072 95 whole, 97 in two)
+      const int slots = a.batch <= per ? per : 2 * per, slots_long = a.batch <= per ? per : 2 * per + 3 * per / 4;
+      const auto up = [&](int n) {
+        return fminf(n >= 2 * a.batch ? 0.5f : 0.25f, 0.97f - (float)(n % a.batch) / (float)a.batch);
+      };
+      // batches of two blocks per CU and more: one part per sequence without the cut (64
+      // sequences: equal lengths 43.2 against 43.6 us, 47-2000 positions 48.1 against 49.4)
+      const SpanRule rule = {(float)slots, up(slots), (float)slots_long, up(slots_long), a.batch < 2 * per};
+      int parts = a.batch;  // with the cut: fewer than two per CU and the extra ones
+      if (rule.cut) parts += min(slots_long, a.batch * (kSpanSplits - 1));
+      hipLaunchKernelGGL(attn_span_kernel, dim3((unsigned)parts * a.kvh), dim3(256), 0, stream, a, rule);
     }
   } else if (a.chunk == kAttnChunk) {
     const int ns = (a.max_ctx + kAttnChunk - 1) / kAttnChunk;

@@ -21,6 +21,12 @@ CASES = [  # lengths, capacity, kv heads
     ([1 + (53 * i) % 704 for i in range(64)], 704, 4),          # every lane a sequence
     ([1 + (37 * i) % 640 for i in range(100)], 640, 4),         # two groups of lanes
     ([576 - 8 * (i % 72) for i in range(64)] + [-3], 576, 8),   # one part each, a position out of range
+    ([101] * 24, 640, 8), ([191, 192, 193, 256, 320, 321, 384, 385], 1024, 8),  # too short to cut, and just not
+    ([1024] * 12, 1024, 8), ([700] * 16, 1024, 8), ([513] * 17, 576, 8),  # equal batches, two parts and one
+    ([4000] + [200 + i for i in range(31)], 4096, 8),           # one long sequence beside short ones
+    ([2624 - i for i in range(36)], 2624, 8),                   # past one block per CU, long enough for two parts
+    ([2600 - 40 * i for i in range(63)], 2624, 8),              # the same, ragged
+    ([640 - 5 * i for i in range(126)] + [641], 640, 4),        # two groups of lanes with extra parts
 ]
 
 
@@ -57,3 +63,28 @@ def test_span_attention_vs_fp64(dev, lengths, cap, kvh):
         np.testing.assert_array_less((out[b].double() - ref).abs().cpu().numpy(), (2.0 ** -16 * size + 1e-7).cpu().numpy())
     status = ws[:4].view(torch.int32).item()
     assert status == (_lib.STATUS_BAD_POSITION if any(not 0 < n <= cap for n in lengths) else 0)
+
+
+@pytest.mark.parametrize("lengths,cap,whole", [
+    ([101] * 24, 640, True), ([150] * 8, 8192, True), ([192, 64, 1], 1024, True),  # a split would save too little
+    ([1024] * 24, 1024, True), ([700] * 20, 2048, True), ([600] * 63, 1024, True),  # about one block per CU already
+    ([1024] * 8, 1024, False), ([8192], 8192, False), ([4000] + [200] * 15, 4096, False), ([640] * 4, 640, False),
+])
+def test_span_attention_splits_where_it_pays(dev, lengths, cap, whole):
+    """Whether any sequence is cut into parts, read from the workspace: a cut leaves its partials there,
+    whole sequences write nothing but their output."""
+    lib = _lib.load()
+    B = len(lengths)
+    kv = KVCache(Qwen3Config(), 1, B, cap, dev)
+    kv.data.normal_()
+    q = torch.randn(B, 16, 128, device=dev)
+    m = Q4dModel(hidden_size=1024, intermediate_size=3072, num_layers=1, num_q_heads=16, num_kv_heads=8,
+                 head_dim=128, vocab_size=2, max_ctx=cap, rms_norm_eps=1e-6, attn_scaling=128 ** -0.5)
+    nbytes = int(lib.q4d_workspace_bytes(ctypes.byref(m), B))
+    ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
+    pos = torch.tensor([n - 1 for n in lengths], dtype=torch.int32, device=dev)
+    out = torch.empty(B, 16, 128, device=dev)
+    kvd = kv.descriptor()
+    check(lib.q4d_cached_attention(ctypes.byref(m), ctypes.byref(kvd), 0, q.data_ptr(), pos.data_ptr(), out.data_ptr(),
+                                   _lib.Q4D_F32, ws.data_ptr(), nbytes, current_stream()), "q4d_cached_attention")
+    assert bool((ws != 0).any()) == (not whole)
