@@ -1118,17 +1118,25 @@ static int launch_gemm_bm(const GemmArgs& a, int ep, bool pair, hipStream_t st) 
 
 // Whether the rows kernel (q4d_rows.hip) runs: asked for, one matrix, and few enough outputs.
 // The tiled kernels' time there is their chain of K steps on too few blocks, whatever M is
-// (K = 1024 / 2048 / 3072: 12-15 / 22-24 / 31-34 us up to the sizes below); the rows kernel
-// splits K over the waves of a block: 64 rows of 3072 x 1024 12.6 -> 5.2 us, of 1024 x 3072
-// 32.7 -> 4.0, 512 rows 14.5 -> 11.9 and 33.8 -> 10.1, 1024 x 1024 x 3072 34.0 -> 18.2.  Both
-// grow with K, so they cross at a number of outputs: 3072 x 1024 between 512 and 768 rows,
-// 2048 x 1024 at 1024, 1024 x 3072 between 1024 and 2048.  Widths other than the projections'
-// take the kernel's general loop, which is slower: up to 64 rows.
-static bool rows_apply(const GemmArgs& a, int ep, bool pair) {
+// (K = 1024 / 2048 / 3072: 13 / 23 / 33 us, with a residual 17 / 27 / 42, up to the sizes
+// below); the rows kernel splits K over the waves of a block: 64 rows of 3072 x 1024 12.6 ->
+// 4.6 us, of 1024 x 3072 32.7 -> 3.8, 512 rows 13.5 -> 11.1 and 33.8 -> 9.4, 1024 x 1024 x 3072
+// 32.4 -> 17.6.  Both grow with K, so they cross at a number of outputs, in whole rounds of its
+// blocks (2048 outputs each, two to a CU).  Two and a half rounds hold at K = 3072 and with a
+// residual (1700 rows of 1024 x 2048 27.0 against 23.4); without one the tiled kernels are
+// faster past one and a half rounds at K = 2048 (1540 rows 23.0 against 28.4; 1530 23.1 against
+// 22.9), and a matrix of few rows crosses earlier (10000 rows of 128 x 2048 25.7 against 26.3,
+// 8000 25.3 against 20.2; 13000 of 128 x 1024 13.4 against 14.7, 12288 13.4 against 12.3).
+// Widths other than the projections' take the kernel's general loop, which is slower: up to 64
+// rows.
+bool rows_apply(const GemmArgs& a, int ep, bool pair) {
   if (!a.rows || pair || a.nseg != 1 || (ep != EP_F16 && ep != EP_F32 && ep != EP_RESID)) return false;
   if (a.ldy != a.N || a.K % 128 || !aligned(a.s[0], 4)) return false;
   if (a.K != 1024 && a.K != 2048 && a.K != 3072) return a.M <= 64;
-  return (long long)a.M * a.N <= 1750000;
+  long long most = 1750000;
+  if (ep != EP_RESID && a.K == 2048) most = a.N < 1024 ? 512 * 2048 : 768 * 2048;
+  if (ep != EP_RESID && a.K == 1024 && a.N < 1024) most = 768 * 2048;
+  return (long long)a.M * a.N <= most;
 }
 
 int launch_gemm(const GemmArgs& a, int ep, bool pair, hipStream_t st) {

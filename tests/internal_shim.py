@@ -36,6 +36,16 @@ int shim_chain_resid(int M, int N, int K, int ksplit) {
   a.part_cap = (size_t)1 << 40;
   return chain_applies(a, EP_RESID, false);
 }
+// q4d_gemm's choice of the rows kernel
+int shim_rows_apply(int M, int N, int K, int ep) {
+  alignas(16) static float memory[4];  // never read
+  GemmArgs a;
+  memset(&a, 0, sizeof(a));
+  a.M = M; a.N = a.ldy = a.seg_end[0] = N; a.K = K;
+  a.nseg = a.rows = 1;
+  a.s[0] = reinterpret_cast<const uint16_t*>(memory);
+  return rows_apply(a, ep, false);
+}
 // launch_gemm as the batched decode step calls it (the skinny kernel at up to 64 rows)
 int shim_skinny_gemm(const q4d_matrix_t* w, int nseg, const uint16_t* x, int M, void* y, int ep, const float* resid,
                      float* part, size_t part_floats, int x_tiled, int y_tiled, int* ksplit_used, void* stream) {
@@ -82,6 +92,7 @@ def load() -> ctypes.CDLL:
     i, p = ctypes.c_int, ctypes.c_void_p
     lib.shim_rows_tile.argtypes, lib.shim_rows_tile.restype = [i, i, i, i, p], None
     lib.shim_chain_resid.argtypes, lib.shim_chain_resid.restype = [i, i, i, i], i
+    lib.shim_rows_apply.argtypes, lib.shim_rows_apply.restype = [i, i, i, i], i
     lib.shim_skinny_gemm.argtypes = [p, i, p, i, p, i, p, p, ctypes.c_size_t, i, i, p, p]
     lib.shim_skinny_gemm.restype = i
     return lib

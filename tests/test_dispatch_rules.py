@@ -38,3 +38,18 @@ def test_chain_resid_needs_a_split():
             for ksplit in (0, 1, 2):
                 applies = internal_shim.load().shim_chain_resid(m, 1024, k, ksplit)
                 assert applies == (ksplit == 2 and k // 2 in (512, 1024, 1536)), (m, k, ksplit)
+
+
+# (rows, N, K, ep): the rows kernel is the faster one / the tiled kernels are, measured next to the lines
+ROWS = [(1, 128, 1024, "F16"), (569, 3072, 1024, "F16"), (1700, 1024, 1024, "F32"), (12288, 128, 1024, "F16"),
+        (1536, 1024, 2048, "F16"), (768, 2048, 2048, "F32"), (8000, 128, 2048, "F16"), (1700, 1024, 2048, "RESID"),
+        (3400, 512, 2048, "RESID"), (13000, 128, 3072, "F32"), (1700, 1024, 3072, "F16"), (64, 128, 1152, "F16")]
+TILED = [(13000, 128, 1024, "F16"), (6800, 256, 1024, "F32"), (1540, 1024, 2048, "F16"), (850, 2048, 2048, "F32"),
+         (425, 4096, 2048, "F16"), (10000, 128, 2048, "F16"), (4500, 256, 2048, "F16"), (2800, 512, 2048, "F32"),
+         (1800, 1024, 1024, "RESID"), (1800, 1024, 3072, "F16"), (65, 128, 1152, "F16"), (4, 128, 1088, "F16")]
+
+
+@pytest.mark.parametrize("calls,rows", [(ROWS, 1), (TILED, 0)], ids=["rows", "tiled"])
+def test_gemm_takes_the_faster_kernel(calls, rows):
+    for m, n, k, ep in calls:
+        assert internal_shim.load().shim_rows_apply(m, n, k, getattr(internal_shim, f"EP_{ep}")) == rows, (m, n, k, ep)
