@@ -817,7 +817,8 @@ int launch_gemv_xp(const GemvArgs& a, int xm, int xp, int ep, bool pair, hipStre
   if ((a.x_parts && !aligned(a.x_parts, 16)) || (a.x_out && !aligned(a.x_out, 16))) return Q4D_ERR_BAD_ADDR;
   if (xm == X_F16 && xp != 1) return Q4D_ERR_DTYPE;
   // plain linear over several rows: one unpacked weight for 16 of them
-  if (a.batch >= kRowsMin && a.nseg == 1 && !pair && (xm == X_F16 || xm == X_F32) && (ep == EP_F16 || ep == EP_F32))
+  if (a.nseg == 1 && !pair && (xm == X_F16 || xm == X_F32) && (ep == EP_F16 || ep == EP_F32) &&
+      rows_linear(a.batch, a.rows, a.cols, xm == X_F32))
     return launch_rows(RowsArgs{a.w[0], a.s[0], a.x, a.y, nullptr, a.batch, a.rows, a.cols}, xm == X_F32, xp, ep, st);
   // unused segments: empty ranges on segment 0's memory, never selected
   GemvArgs b = a;
@@ -848,7 +849,7 @@ int launch_gemv_group(int rows, int cols, int batch, const uint8_t* const* w, co
     if (!w[i] || !s[i] || !x[i] || !y[i]) return Q4D_ERR_NULL;
     if (!aligned(w[i], 16) || !aligned(s[i], 4) || !aligned(x[i], 16)) return Q4D_ERR_BAD_ADDR;
   }
-  if (batch >= kRowsMin)  // as q4d_linear
+  if (rows_linear(batch, rows, cols, xm == X_F32))  // as q4d_linear, so that the bits are its
     return launch_rows_group(batch, rows, cols, w, s, x, y, count, xm == X_F32, xp, ep, st);
   GemvGroupArgs G;
   memset(&G, 0, sizeof(G));

@@ -223,10 +223,16 @@ struct RowsTile {
   bool k12;
 };
 RowsTile rows_tile(int M, int N, int K, int count);
-// Activation rows from which q4d_linear takes this kernel instead of one GEMV per row
-// (3072 x 1024 / 1024 x 3072, fp32: 3 rows 3.7 / 4.5 us as GEMVs; 4 rows 4.0 / 5.0 against
-// 3.2 / 5.1 here, 8 rows 5.8 / 8.0 against 3.2 / 5.1).
-constexpr int kRowsMin = 4;
+// Whether q4d_linear and q4d_linear_group take this kernel instead of a GEMV per row: from 4
+// activation rows on (3 rows of 3072 x 1024 3.7 us as GEMVs), where the outputs are enough.  Few
+// outputs are bound by one memory round trip and a block's own work, which is longer here (LDS
+// staging of 16 rows, a sum over 8 waves); the GEMVs' time grows with their number.  us as GEMVs
+// / here, fp32: 4 rows of 64 x 3072 3.0 / 4.8, of 1024 x 1024 2.7 / 2.9, of 1024 x 3072 4.9 / 4.9,
+// 5 of 1024 x 1024 3.0 / 2.9, 6 of 1024 x 2048 4.8 / 4.1; fp16: 5 of 1024 x 1024 2.56 / 2.58, 6
+// 2.58 / 2.56, 4 of 1024 x 3072 3.7 / 3.7, 5 of 1024 x 2048 3.4 / 3.0.
+inline bool rows_linear(int batch, int rows, int K, bool xf32) {
+  return batch >= 4 && (long long)batch * rows >= (xf32 ? (K == 3072 ? 3800 : 4097) : (K == 1024 ? 6144 : 3500));
+}
 
 // ---- other launchers ---------------------------------------------------------
 int launch_rms_norm(const float* x, const float* gamma, float eps, int rows, int dim, void* y,

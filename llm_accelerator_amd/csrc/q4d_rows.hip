@@ -1,6 +1,6 @@
 // Q4 linear over several activation rows on MFMA, at the GEMV's precision (gfx950).
 //
-//   y[m, n] = sum_g scale[n, g] * sum_{k in group g} q[n, k] x[m, k]      (4 rows and more)
+//   y[m, n] = sum_g scale[n, g] * sum_{k in group g} q[n, k] x[m, k]      (4 rows and more: rows_linear)
 //
 // The GEMV (q4d_gemv.hip) reads and unpacks every weight again for each activation row: at
 // 211 rows of a 1024 x 3072 matrix its VALU work took 161 us.  Here 16 rows share each
@@ -366,11 +366,10 @@ int launch_rows(const RowsArgs& a, bool xf32, int xp, int ep, hipStream_t st) {
   }
 }
 
-// 64 fp32 matrices, us a call at 4 / 16 / 64 rows (a launch per matrix: 180-206 at K = 1024,
-// 317-380 at 3072, bound by the host; the grouped GEMV, which reads and unpacks a matrix again
-// for each row): 128 x 1024 5.0 / 6.5 / 11.1 (GEMV 5.5 / 13.8 / 47), 1024 x 1024 13.7 / 16.4 /
-// 50.7 (25 / 89 / 318), 3072 x 1024 32 / 35 / 125 (70 / 239 / 951), 1024 x 3072 35 / 41 / 133
-// (100 / 370 / 1469).
+// 64 fp32 matrices, us a call (a launch per matrix: 190-350, bound by the host; in brackets the
+// grouped GEMV, which reads and unpacks a matrix again for each row): 1024 x 1024 at 8 / 16 / 64
+// rows 14.4 / 16.3 / 52 (47 / 88 / 317), 3072 x 1024 at 4 / 16 / 64 rows 33 / 35 / 125 (70 / 239
+// / 951), 1024 x 3072 at 4 / 16 / 64 rows 35 / 42 / 137 (98 / 370 / 1467).
 int launch_rows_group(int M, int N, int K, const uint8_t* const* w, const uint16_t* const* s, const void* const* x,
                       void* const* y, int count, bool xf32, int xp, int ep, hipStream_t st) {
   if (count <= 0 || !xp || (ep != EP_F16 && ep != EP_F32)) return Q4D_ERR_SHAPE;

@@ -36,7 +36,8 @@ int shim_chain_resid(int M, int N, int K, int ksplit) {
   a.part_cap = (size_t)1 << 40;
   return chain_applies(a, EP_RESID, false);
 }
-// q4d_gemm's choice of the rows kernel
+// q4d_linear's and q4d_gemm's choice of the rows kernel
+int shim_rows_linear(int batch, int rows, int K, int xf32) { return rows_linear(batch, rows, K, xf32); }
 int shim_rows_apply(int M, int N, int K, int ep) {
   alignas(16) static float memory[4];  // never read
   GemmArgs a;
@@ -92,6 +93,7 @@ def load() -> ctypes.CDLL:
     i, p = ctypes.c_int, ctypes.c_void_p
     lib.shim_rows_tile.argtypes, lib.shim_rows_tile.restype = [i, i, i, i, p], None
     lib.shim_chain_resid.argtypes, lib.shim_chain_resid.restype = [i, i, i, i], i
+    lib.shim_rows_linear.argtypes, lib.shim_rows_linear.restype = [i, i, i, i], i
     lib.shim_rows_apply.argtypes, lib.shim_rows_apply.restype = [i, i, i, i], i
     lib.shim_skinny_gemm.argtypes = [p, i, p, i, p, i, p, p, ctypes.c_size_t, i, i, p, p]
     lib.shim_skinny_gemm.restype = i

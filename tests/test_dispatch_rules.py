@@ -53,3 +53,14 @@ TILED = [(13000, 128, 1024, "F16"), (6800, 256, 1024, "F32"), (1540, 1024, 2048,
 def test_gemm_takes_the_faster_kernel(calls, rows):
     for m, n, k, ep in calls:
         assert internal_shim.load().shim_rows_apply(m, n, k, getattr(internal_shim, f"EP_{ep}")) == rows, (m, n, k, ep)
+
+
+def test_linear_takes_the_faster_kernel():
+    """A GEMV per row up to 3 rows and for few outputs, the rows kernel past that."""
+    gemv = [(3, 3072, 1024, 1), (4, 64, 3072, 1), (100, 2, 2048, 1), (4, 1024, 1024, 1), (4, 1024, 1024, 0),
+            (5, 1024, 1024, 0), (33, 64, 2048, 1), (6, 512, 3072, 0), (3, 151936, 1024, 0)]
+    rows = [(5, 1024, 1024, 1), (6, 1024, 1024, 0), (4, 2048, 1024, 1), (4, 1024, 2048, 0), (4, 1024, 3072, 0), (4, 1024, 3072, 1),
+            (33, 130, 3072, 1), (65535, 2, 1024, 1), (4, 151936, 1024, 1)]
+    for calls, want in ((gemv, 0), (rows, 1)):
+        for c in calls:
+            assert internal_shim.load().shim_rows_linear(*c) == want, c

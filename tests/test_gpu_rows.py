@@ -1,4 +1,4 @@
-"""q4d_linear over several activation rows (the MFMA kernel of 4 rows and more) on the GPU
+"""q4d_linear over several activation rows (the MFMA kernel, from 4 rows and some 4000 outputs on) on the GPU
 vs the oracle: tile edges in both directions, every matrix width, every input and output type."""
 
 import ctypes
@@ -19,7 +19,10 @@ ACC = 4e-6  # fp32 accumulation error relative to sum |w x|, the bar of the one-
 
 
 @pytest.mark.parametrize("m,n,k,xdtype,ydtype,precision", [
-    (4, 2, 1024, torch.float32, Q4D_F32, 2),         # one tile, nearly empty
+    (4, 2, 1024, torch.float32, Q4D_F32, 2),         # few outputs: a GEMV per row
+    (4, 1026, 1024, torch.float32, Q4D_F32, 2),      # the first past the GEMVs: one row tile, nearly empty
+    (4, 1024, 1024, torch.float32, Q4D_F32, 2),      # ... and the last of them
+    (6, 1024, 1024, torch.float16, Q4D_F32, 1),
     (16, 1024, 2048, torch.float32, Q4D_F32, 2),     # one row tile, one weight tile per block
     (17, 1030, 1024, torch.float16, Q4D_F16, 1),     # ragged both ways, fp16 in and out
     (33, 3072, 3072, torch.float32, Q4D_F32, 2),     # two weight tiles per block
@@ -71,7 +74,7 @@ def test_linear_rows_integer_exact(dev, m, n, k):
 def test_linear_rows_one_bad_row_stays_alone(dev):
     """A row holding an infinity or a NaN does not reach the other rows of its tile."""
     rng = np.random.default_rng(3)
-    w = q4(rng.integers(0, 256, size=(64, 512), dtype=np.uint8), np.full((64, 16), 100, dtype=np.uint16), dev)
+    w = q4(rng.integers(0, 256, size=(256, 512), dtype=np.uint8), np.full((256, 16), 100, dtype=np.uint16), dev)
     x = torch.randn(20, 1024, device=dev)
     clean = linear(w, x)
     x[5, 17], x[9, 1000] = float("inf"), float("nan")
@@ -98,9 +101,10 @@ def test_linear_group_rows_equal_single_calls(dev):
 
 
 @pytest.mark.parametrize("m,n,k,count,xdtype,ydtype,precision", [
-    (4, 130, 1024, 70, torch.float32, Q4D_F32, 2),      # 64 + 6: four weight tiles per block, then one
+    (16, 258, 1024, 70, torch.float32, Q4D_F32, 2),     # 64 + 6: four weight tiles per block, then one
+    (4, 130, 1024, 70, torch.float32, Q4D_F32, 2),      # few outputs: the grouped GEMV
     (5, 1026, 3072, 64, torch.float32, Q4D_F16, 2),     # four weight tiles per block, the waves of one
-    (20, 66, 3072, 2, torch.float32, Q4D_F32, 2),       # one tile, 12 waves
+    (20, 258, 3072, 2, torch.float32, Q4D_F32, 2),      # one tile, 12 waves
     (33, 3072, 3072, 3, torch.float32, Q4D_F32, 2),     # two weight tiles alone, two row tiles together
     (40, 512, 2048, 65, torch.float16, Q4D_F16, 1),     # 64 + 1: the last a launch of its own
     (17, 512, 3072, 66, torch.float32, Q4D_F32, 1),
@@ -108,7 +112,7 @@ def test_linear_group_rows_equal_single_calls(dev):
     (70, 130, 2048, 64, torch.float32, Q4D_F32, 2),     # two row tiles, the general loop
 ])
 def test_linear_group_rows_one_launch_and_bits(dev, m, n, k, count, xdtype, ydtype, precision):
-    """q4d_linear_group at 4 rows and more: one launch per 64 matrices (the kernels a captured call
+    """q4d_linear_group over several rows: one launch per 64 matrices (the kernels a captured call
     records), and each output equals its own q4d_linear call bit for bit whatever tile the group takes."""
     from llm_accelerator_amd.model import current_stream
     lib = _lib.load()
