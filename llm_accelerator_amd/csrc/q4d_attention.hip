@@ -494,6 +494,11 @@ __device__ __forceinline__ SpanWork span_extra(const AttnArgs& a, int idx, const
   }
 }
 
+// a = a b + c where a is (left alone, the loop adds into c's register and copies it back).
+__device__ __forceinline__ void fma_into(float& a, float b, float c) {
+  asm("v_fma_f32 %0, %0, %1, %2" : "+v"(a) : "v"(b), "v"(c));
+}
+
 // Long-context variant of attn_kernel<64> with merge = 1 (batched decode,
 // q4d_cached_attention): a block covers one of a sequence's nsplit nearly equal
 // parts of its T = pos + 1 positions (parts of whole 64-position sub-chunks) as
@@ -508,11 +513,10 @@ __device__ __forceinline__ SpanWork span_extra(const AttnArgs& a, int idx, const
 // parts 6.27; one block per head with 64-position sub-chunks 5.48).
 // The parts are cut from the sequences' own positions (SpanRule).  Cut from the capacity
 // instead, one long part held up ragged batches and short contexts of a large cache ran on few
-// blocks (us a call, from the capacity / now): 24 x 649-1500 positions of 2048 25.9 / 23.5, 8 x
-// 2048 of 8192 31.7 / 14.5, 40 x 2048 of 4096 79 / 62, one sequence of 8191 18.7 / 14.1; equal
-// batches that fill the cache are within 3 % (one of 952 of 1024 6.8 / 7.1), 24 x 4095 of 4096
-// 75 / 64.  The first parts' loads go out before the cut is known, which hides its ~0.4 us from
-// the sequences that stay whole.
+// blocks (us a call, from the capacity / now): 24 x 649-1500 positions of 2048 25.5 / 22.6, 8 x
+// 2048 of 8192 31.7 / 13.9, 40 x 2048 of 4096 79 / 59, one sequence of 8191 18.7 / 14.1, 24 x
+// 4095 of 4096 75 / 61; none of 281 batches is more than 3 % slower.  The first parts' loads go
+// out before the cut is known, which hides its ~0.4 us from the sequences that stay whole.
 // Same prologue and partial format as attn_kernel<64>; thread t owns dims
 // 8 (t % 16) .. +7 of positions t / 16 + 16 i.
 __global__ __launch_bounds__(256) void attn_span_kernel(const AttnArgs a, const SpanRule rule) {
@@ -693,28 +697,29 @@ __global__ __launch_bounds__(256) void attn_span_kernel(const AttnArgs a, const 
     m0 = rows_max(m0);
     m1 = rows_max(m1);
     const float Mn0 = fmaxf(M0, m0), Mn1 = fmaxf(M1, m1);
+    // (v_exp itself: weights under 2^-126 of the running maximum's are 0; exp2f's care for them
+    // is 50 of the loop's 370 instructions)
     float e0[NPT], e1[NPT], s0 = 0.f, s1 = 0.f;
 #pragma unroll
     for (int i = 0; i < NPT; ++i) {
       const bool ok = pr + 16 * i < n;
-      e0[i] = ok ? exp2f(y0[i] - Mn0) : 0.f;
-      e1[i] = ok ? exp2f(y1[i] - Mn1) : 0.f;
+      e0[i] = ok ? __builtin_amdgcn_exp2f(y0[i] - Mn0) : 0.f;
+      e1[i] = ok ? __builtin_amdgcn_exp2f(y1[i] - Mn1) : 0.f;
       s0 += e0[i];
       s1 += e1[i];
     }
     s0 = rows_sum(s0);
     s1 = rows_sum(s1);
-    const float sc0 = M0 == -INFINITY ? 0.f : exp2f(M0 - Mn0);
-    const float sc1 = M1 == -INFINITY ? 0.f : exp2f(M1 - Mn1);
+    const float sc0 = M0 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M0 - Mn0);
+    const float sc1 = M1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M1 - Mn1);
     L0 = fmaf(L0, sc0, s0);
     L1 = fmaf(L1, sc1, s1);
     M0 = Mn0;
     M1 = Mn1;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      o0[e] *= sc0;
-      o1[e] *= sc1;
-    }
+    // the sub-chunk's sum by itself, then onto the running one, which so is rounded once a
+    // sub-chunk (error of 24 x 649-1500 positions as whole sequences 2.1e-7 -> 1.7e-7, 1.8e-7 in
+    // two and three parts)
+    float t0[8], t1[8];
 #pragma unroll
     for (int i = 0; i < NPT; ++i) {
       const int p = pr + 16 * i;
@@ -723,9 +728,14 @@ __global__ __launch_bounds__(256) void attn_span_kernel(const AttnArgs a, const 
       unpack8(vq, vf);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        o0[e] = fmaf(e0[i], vf[e], o0[e]);
-        o1[e] = fmaf(e1[i], vf[e], o1[e]);
+        t0[e] = fmaf(e0[i], vf[e], i ? t0[e] : 0.f);
+        t1[e] = fmaf(e1[i], vf[e], i ? t1[e] : 0.f);
       }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      fma_into(o0[e], sc0, t0[e]);
+      fma_into(o1[e], sc1, t1[e]);
     }
 #pragma unroll
     for (int i = 0; i < NPT; ++i) {
