@@ -180,7 +180,11 @@ int q4d_read_status(const void* ws, size_t ws_bytes, const q4d_model_t* model, i
 
 /* ---- primitive ops ------------------------------------------------------- */
 /* y[m, :] = W x[m, :] for m < batch.  x: [batch, cols] (x_dtype), y: [batch, rows] (y_dtype).
- * Supported cols: 1024, 2048, 3072; rows even. */
+ * Supported cols: 1024, 2048, 3072; rows even.  Deterministic: one call's shape and inputs
+ * give the same bits every time.  The order of the fp32 sums follows the shape: up to 3 rows
+ * and for few outputs (about 4000) each row is a GEMV by itself, past that the rows share an
+ * MFMA kernel, at cols = 3072 with two splits of the sum by batch and rows.  So a row's last
+ * bits may depend on `batch`, though not on the other rows' values. */
 int q4d_linear(const q4d_matrix_t* w, const void* x, int32_t x_dtype, void* y, int32_t y_dtype,
                int32_t batch, void* stream);
 /* No counterpart in the reference (it applies one matrix per call,
@@ -233,7 +237,10 @@ int q4d_causal_attention(const float* q, const float* k, const float* v, float* 
 int q4d_kv_append(const q4d_kv_cache_t* kv, int32_t layer, const float* k, const float* v,
                   const int32_t* positions, int32_t* status, void* stream);
 /* GQA decode attention over cache positions [0, positions[b]] of `layer`.
- * q: fp32 [batch, q_heads, head_dim] already normed/roped; out: fp16 [batch, q_heads*head_dim]. */
+ * q: fp32 [batch, q_heads, head_dim] already normed/roped; out: [batch, q_heads*head_dim] in
+ * out_dtype.  Past max_ctx = 512 a sequence's positions may be cut into parts whose number
+ * follows from the whole batch's positions, so its last bits (fp32 rounding) may depend on the
+ * lengths of the other sequences, though not on their values. */
 int q4d_cached_attention(const q4d_model_t* model, const q4d_kv_cache_t* kv, int32_t layer,
                          const float* q, const int32_t* positions, void* out, int32_t out_dtype,
                          void* ws, size_t ws_bytes, void* stream);
@@ -257,16 +264,19 @@ int q4d_lm_head_argmax_batch(const q4d_model_t* model, const float* hidden, int3
 /* y[m, :] = W x[m, :] for m < M on MFMA, for many activation rows sharing the weights
  * (prefill, batched decode): x fp16 [M, cols]; y [M, rows] in y_dtype; if resid is not
  * NULL, y (fp32) = resid + W x (resid may alias y).  Q4 tiles are dequantised to fp16
- * (one rounding of q*scale) and accumulated in fp32.  rows % 128 == 0, cols % 64 == 0. */
+ * (one rounding of q*scale) and accumulated in fp32.  rows % 128 == 0, cols % 64 == 0.
+ * The order of the fp32 sums follows the shape (few outputs, M x rows up to 1-1.75 M: K split
+ * over a block's waves; more: one chain over K), so a row's last bits may depend on M, though
+ * not on the other rows' values. */
 int q4d_gemm(const q4d_matrix_t* w, const uint16_t* x, int32_t M, void* y, int32_t y_dtype,
              const float* resid, void* stream);
-/* q4d_gemm with the K dimension split over `ksplit` blocks per output tile
- * (1..16, at most cols / 64; 0 = chosen for the shape), for few activation
- * rows where the output tiles alone leave the device idle: each split's fp32
- * tile goes to `part` (ksplit x M x rows floats, 16-byte aligned), then the
- * splits are added in order.  Same result as q4d_gemm up to the grouping of
- * the fp32 sums.  No counterpart in the reference; it is the batched-decode
- * projection path of q4d_decode_batch, exported for callers with scratch. */
+/* q4d_gemm with a partial buffer for a split of K over `ksplit` blocks per output tile
+ * (1..16, at most cols / 64), for few activation rows where the output tiles alone leave the
+ * device idle: each split's fp32 tile goes to `part` (ksplit x M x rows floats, 16-byte
+ * aligned), then the splits are added in order.  ksplit = 0 chooses for the shape: for few
+ * outputs the kernel of q4d_gemm, which splits K inside a block and leaves `part` alone; past
+ * that the batched-decode kernel at M <= 64 or a number of splits, which may use it.  Same
+ * result as q4d_gemm up to the grouping of the fp32 sums.  No counterpart in the reference. */
 int q4d_gemm_splitk(const q4d_matrix_t* w, const uint16_t* x, int32_t M, void* y, int32_t y_dtype,
                     const float* resid, float* part, size_t part_bytes, int32_t ksplit, void* stream);
 
@@ -342,7 +352,9 @@ int q4d_run_one_token_noalloc(const q4d_model_t* model, const int32_t* tokens, c
  * positions[b] (device int32 [batch], each sequence its own position) through embedding,
  * all layers (projections as MFMA GEMMs over the batch, GQA attention per sequence) and the
  * LM head; writes next_tokens[b], scores[b] and, if logits is not NULL, logits
- * [batch, vocab] (fp32).  Activations enter each projection as fp16.  The KV cache must
+ * [batch, vocab] (fp32).  Activations enter each projection as fp16.  A sequence's logits do
+ * not depend on the other sequences' values, but their last bits may on the batch's size and,
+ * past max_ctx = 512, on the other positions (q4d_cached_attention).  The KV cache must
  * have batch >= `batch`; the workspace is sized by q4d_workspace_bytes(model, batch).
  * No counterpart in the reference (its decode is batch 1); per sequence it computes
  * run_manual_one_token (10_validate_full_run_one_token.py:17-56). */

@@ -11,10 +11,11 @@
 // of every block take neighbours, then the next pair of waves): the waves that take one more
 // are spread over the CUs, and the two 64-byte halves of a line of logits meet in one L2.
 //
-// What bounds it (24 / 64 rows, kernel and argmax rows together, was 64.4 / 73.5 us with the
-// norm's launch): 40 / 59 us; with the activations' LDS reads taken out 34 / 42, without the
-// logits' stores 37 / 52, with neither, the unpacking nor the argmax 26.5.  Two table tiles per
-// read of the activations took 40 / 64: fewer, longer steps per wave cost what they save.
+// What bounds it (24 / 64 rows, a call among others with its argmax rows 35 / 57 us, 65 / 71 on
+// the tiled GEMM with the norm's launch): of the time, the activations' LDS reads are about 15 /
+// 29 %, the logits' stores 8 / 12 %; without either, the unpacking and the argmax two thirds are
+// left at 24 rows.  Two table tiles per read of the activations took as long at 24 rows and 8 %
+// longer at 64: fewer, longer steps per wave cost what they save.
 //
 // The products and their order are the tiled kernel's: fp16 operands (weights rounded once),
 // 32 columns per MFMA in order, fp32 accumulation.
@@ -183,7 +184,7 @@ int launch_lm_batch(const LmBatchArgs& a, int* nparts, hipStream_t st) {
   const int blocks = min(device_cus(), a.N / 128);
   *nparts = blocks;
   // waves per block: as many as the registers allow, where that measured faster
-  // (24 rows: 40.0 us with 16, 41.5 with 8; 16 rows: 32.2 with 8, 34.6 with 16)
+  // (24 rows: 4 % slower with 8 than with 16; 16 rows: 7 % slower with 16 than with 8)
   const auto go = [&](auto kernel, int nw) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * nw), 0, st, a); };
   switch ((a.M + 15) / 16) {
     case 1: go(lm_batch_kernel<1, 8>, 8); break;

@@ -3,7 +3,7 @@
 //   y[m, n] = sum_g scale[n, g] * sum_{k in group g} q[n, k] x[m, k]      (4 rows and more: rows_linear)
 //
 // The GEMV (q4d_gemv.hip) reads and unpacks every weight again for each activation row: at
-// 211 rows of a 1024 x 3072 matrix its VALU work took 161 us.  Here 16 rows share each
+// 211 rows of a 1024 x 3072 matrix its VALU work took 142 us.  Here 16 rows share each
 // unpacked weight.  The arithmetic keeps the GEMV's precision: the int4 codes enter the MFMA
 // as exact fp16 integers, fp32 activations as an fp16 hi + fp16 lo pair (~22 significant
 // bits, two MFMAs; fp16 activations and activation precision 1 take one), products are
@@ -19,8 +19,8 @@
 // lane, transposed across the four lane rows as in the skinny GEMM (q4d_gemm.hip).
 //
 // What bounds it: a few rows, the launch and one memory round trip (16 rows of 3072 x 1024
-// fp32: 3.2 us, 9.4 as 16 GEMVs); many, the unpacking and splitting VALU work per MFMA and
-// the activations' re-reads from L2 (211 rows of 1024 x 3072: 9.1 us, was 142; 1024 rows of
+// fp32: 3.1 us, 9.4 as 16 GEMVs); many, the unpacking and splitting VALU work per MFMA and
+// the activations' re-reads from L2 (211 rows of 1024 x 3072: 8.6 us, was 142; 1024 rows of
 // 3072 x 1024: 32 us, was 466).
 #include <type_traits>
 
